@@ -1,0 +1,56 @@
+"""The standalone operations whose rows are split over several workgroups, at the edges of their
+parts."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("B,V", [(3, 2048), (3, 2049), (2, 8191), (2, 8192), (3, 8193), (2, 16385),
+                                 (130, 32001), (1, 524288)])
+def test_softmax_parts(cuda, dtype, B, V):
+    """Parts of a row (8192 elements at most, odd row starts, the smallest and largest row) against
+    float64: |y - max| <= 80 rounds by 80 * 2^-24 = 4.8e-6 in a term and, averaged, in the sum
+    (rtol 1e-5).  One row has a part of -inf, one a NaN, one +inf (its probabilities are NaN)."""
+    import torch
+
+    from vllm_webgpu_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(V)
+    x = torch.randn((B, V), generator=g, device=cuda) * 3
+    if B > 1:
+        x[0, : V // 2] = -float("inf")
+        x[1, V - 1] = float("nan")
+    if B > 2:
+        x[2, V // 3] = float("inf")
+    x = x.to({"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype])
+    T = torch.linspace(0.7, 1.3, B, device=cuda)
+    p, rm, ls = ops.softmax(x, T)
+    y = (x.float() / T[:, None]).double()
+    m = torch.nan_to_num(y, nan=-float("inf"), posinf=float("inf")).amax(1)
+    assert torch.equal(rm.double(), m)
+    e = torch.nan_to_num(torch.exp(y - m[:, None]), nan=0.0)
+    ok = torch.isfinite(m)
+    S = e.sum(1)
+    torch.testing.assert_close(p[ok].double(), (e / S[:, None])[ok], rtol=1e-5, atol=1e-12)
+    torch.testing.assert_close(ls[ok].double(), S[ok].log(), rtol=1e-6, atol=5e-6)
+    if B > 2:
+        assert torch.isnan(p[2]).all() and ls[2] == -float("inf")
+
+
+@pytest.mark.parametrize("V", [20000, 50000])
+def test_softmax_over_its_logits(cuda, V):
+    """Probabilities written over the logits (the C entry accepts the same buffer twice) are those
+    of separate buffers: the same elements and exponentials, S summed in another order (1e-6)."""
+    import torch
+
+    from vllm_webgpu_amd import _lib, ops
+
+    x = torch.randn((5, V), device=cuda) * 3
+    want, _, _ = ops.softmax(x)
+    _lib.check(_lib.lib().vws_softmax(x.data_ptr(), _lib.DTYPE_F32, 5, V, V, None, x.data_ptr(), None,
+                                      None, torch.cuda.current_stream().cuda_stream))
+    torch.testing.assert_close(x, want, rtol=1e-6, atol=1e-12)

@@ -20,6 +20,10 @@ template <typename T, bool LP, int XF> __global__ void row_kernel(const void*, i
 template <typename T> __global__ void argmax_kernel(const T*, int64_t, int, int32_t*);
 template <typename T>
 __global__ void softmax_kernel(const T*, int64_t, int, const float*, float*, float*, float*);
+template <typename T>
+__global__ void softmax_part_kernel(const T*, int64_t, int, int, int, const float*, float*);
+template <typename T>
+__global__ void softmax_write_kernel(const T*, int64_t, int, int, int, const float*, float*, float*, float*);
 __global__ void penalties_kernel(KArgs, float*);
 __global__ void selftest_kernel(int, uint32_t, uint32_t, unsigned long long*);
 __global__ void fill_u32_kernel(uint32_t*, size_t, uint32_t);
@@ -302,6 +306,33 @@ KArgs make_kargs(int B, int V, const void* logits, int64_t stride, void* ws, int
     return k;
 }
 
+// Rows of up to kSmRowMax elements take one workgroup each, longer ones parts of at most
+// kSmPartMax: two launches, but every compute unit at work and no thread with more than 32
+// elements.  Measured, one workgroup per row against parts (fp32, a call): 1 x 5000 13.4 and
+// 11.7 us (the host's part), 1024 x 2500 51 and 18 us, 1024 x 32000 102 and 77 us (there the one
+// workgroup holds its row in registers), 32 x 128256 95.5 and 15.8 us, 256 x 128256 109 and 76 us.
+// Probabilities that overlap the logits take one workgroup per row: the parts' partial results
+// lie in the probabilities while other parts still read their logits.
+template <typename T>
+void softmax_launch(const T* logits, int B, int V, int64_t stride, const float* temperature, float* probs,
+                    float* row_max, float* log_sum, hipStream_t s) {
+    const int K = VWS_KERNEL_SOFTMAX;
+    const uintptr_t l0 = reinterpret_cast<uintptr_t>(logits), l1 = l0 + ((size_t)(B - 1) * stride + V) * sizeof(T);
+    const uintptr_t p0 = reinterpret_cast<uintptr_t>(probs), p1 = p0 + (size_t)B * V * sizeof(float);
+    const bool overlap = l0 < p1 && p0 < l1;
+    if (overlap || V <= kSmRowMax) {
+        launch(K, softmax_kernel<T>, dim3(B), dim3(1024), s, logits, stride, V, temperature, probs, row_max, log_sum);
+        return;
+    }
+    // parts of a multiple of 64 elements; the last one holds at least V / n - 63 (n - 1) of
+    // them, more than the 3 n words of the partial results its slice carries
+    const int n = (V + kSmPartMax - 1) / kSmPartMax;
+    const int len = ((V + n - 1) / n + 63) / 64 * 64;
+    launch(K, softmax_part_kernel<T>, dim3(B * n), dim3(kSmThreads), s, logits, stride, V, len, n, temperature, probs);
+    launch(K, softmax_write_kernel<T>, dim3(B * n), dim3(kSmThreads), s, logits, stride, V, len, n, temperature, probs,
+           row_max, log_sum);
+}
+
 }  // namespace
 
 extern "C" {
@@ -547,16 +578,12 @@ int vws_softmax(const void* logits, int32_t dtype, int32_t batch, int32_t vocab,
     if (st) return st;
     if (!probs) return fail(VWS_ERR_INVALID_ARGUMENT, "probs is NULL");
     hipStream_t s = (hipStream_t)stream;
-    const int K = VWS_KERNEL_SOFTMAX;
     if (dtype == VWS_DTYPE_F32)
-        launch(K, softmax_kernel<float>, dim3(batch), dim3(1024), s,
-               static_cast<const float*>(logits), row_stride, vocab, temperature, probs, row_max, log_sum);
+        softmax_launch(static_cast<const float*>(logits), batch, vocab, row_stride, temperature, probs, row_max, log_sum, s);
     else if (dtype == VWS_DTYPE_BF16)
-        launch(K, softmax_kernel<uint16_t>, dim3(batch), dim3(1024), s,
-               static_cast<const uint16_t*>(logits), row_stride, vocab, temperature, probs, row_max, log_sum);
+        softmax_launch(static_cast<const uint16_t*>(logits), batch, vocab, row_stride, temperature, probs, row_max, log_sum, s);
     else
-        launch(K, softmax_kernel<_Float16>, dim3(batch), dim3(1024), s,
-               static_cast<const _Float16*>(logits), row_stride, vocab, temperature, probs, row_max, log_sum);
+        softmax_launch(static_cast<const _Float16*>(logits), batch, vocab, row_stride, temperature, probs, row_max, log_sum, s);
     if ((st = check_launch("vws_softmax"))) return st;
     return ok();
 }

@@ -19,6 +19,13 @@ constexpr int kMergeCap = kFastWaves * kCapW;     // entries the last part can m
 constexpr int kPartMax = 32768;                   // elements per part
 constexpr int kMaxParts = 16;                    // parts per row: VWS_MAX_VOCAB / kPartMax
 
+// Split softmax (vws_ops.hip): threads per part, most elements of a part (32 per thread, kept in
+// registers) and most parts of a row (VWS_MAX_VOCAB / kSmPartMax; one lane of a wave each).
+constexpr int kSmThreads = 256;
+constexpr int kSmPartMax = 32 * kSmThreads;
+constexpr int kSmMaxParts = 64;
+constexpr int kSmRowMax = 2048;  // longest row that one workgroup takes
+
 // General path (one workgroup per row, multi-pass).
 constexpr int kGenThreads = 1024;
 constexpr int kGenWaves = kGenThreads / 64;

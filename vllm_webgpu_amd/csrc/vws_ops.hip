@@ -60,14 +60,24 @@ __global__ __launch_bounds__(kOpThreads) void argmax_kernel(const T* logits, int
     }
 }
 
-// probs = exp_det(x/T - m) / S, m = max x/T, S = sum exp_det(x/T - m); one workgroup per row.
-// Rows of up to 32 values per thread (V <= 32768: 8 chunks of fp32, 4 of 16-bit values) are
-// read once: each thread keeps its chunks in registers through the max, the sum and the write
-// (one read and one write of the row).  Longer rows are read twice: the maximum and S together
-// (an online merge of per-thread running maxima and sums), then the write.  S is summed in
-// double, in a different order than the sequential oracle (and, for long rows, with rescaled
-// partial sums); each probability is e * fl64(1 / S): the probabilities agree with the oracle's
-// to within a few fp32 ulps.
+// probs = exp_det(x/T - m) / S, m = max x/T, S = sum exp_det(x/T - m), S in double.  Two forms,
+// chosen by the launcher (vws_softmax):
+//
+// softmax_kernel, one workgroup per row (short rows, and calls whose probabilities overlap their
+// logits): rows of up to 32 values per thread (V <= 32768 less the two unaligned edges) are read
+// once and written once, each thread keeping its chunks in registers through the max, the sum
+// and the write.  Longer rows are read twice: the maximum and S together (an online merge of
+// per-thread running maxima and sums), then the write.
+//
+// softmax_part_kernel + softmax_write_kernel, several workgroups per row (any V): the first
+// leaves each part's maximum and its sum relative to that maximum, the second combines a row's
+// parts and writes the probabilities.  A row on one CU is bound by that CU's share of the
+// bandwidth and by its issue slots (a division and two exponentials per element), so a batch
+// smaller than the chip needs its rows split: 32 x 128256 fp32 95.5 -> 15.8 us.
+//
+// S is summed in another order than the sequential oracle (and, split, from rescaled partial
+// sums); each probability is e * fl64(1 / S): the probabilities agree with the oracle's to
+// within a few fp32 ulps.
 template <typename T>
 __global__ __launch_bounds__(kOpThreads) void softmax_kernel(const T* logits, int64_t stride, int V,
                                                               const float* temperature, float* probs,
@@ -184,6 +194,143 @@ __global__ __launch_bounds__(kOpThreads) void softmax_kernel(const T* logits, in
     }
 }
 
+// ---- the split softmax -------------------------------------------------------------------
+
+// A thread's elements of part p of a row, in registers: kPartVecs body vectors, then one edge
+// element (the unaligned head and tail together hold fewer than 2 VEC elements, one per thread
+// from thread 0 on).  Everything outside the part is NaN.
+template <typename T>
+struct SoftmaxPart {
+    static constexpr int VEC = Elem<T>::kVec;
+    static constexpr int kVecs = kSmPartMax / (kSmThreads * VEC);
+    int lo, hi, a, nbody, edge;  // edge: this thread's edge element, or -1
+    float v[kVecs][VEC];
+    float ve;
+    __device__ __forceinline__ void load(const T* row, int V, int part_len, int p, float Tt) {
+        lo = p * part_len;
+        hi = min(V, lo + part_len);
+        Slice<T> sl;
+        sl.init(row, lo, hi);
+        a = sl.a;
+        nbody = sl.nbody;
+        const int tid = threadIdx.x;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(row + a, 16u * (uint32_t)nbody);
+#pragma unroll
+        for (int q = 0; q < kVecs; ++q) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rs, 16u * (uint32_t)(q * kSmThreads + tid), 0u, 0);
+            Elem<T>::from_words((uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2], (uint32_t)w[3], v[q]);
+        }
+        const int head = a - lo, tail = hi - sl.body_end();
+        edge = tid < head ? lo + tid : (tid - head < tail ? sl.body_end() + (tid - head) : -1);
+        ve = edge >= 0 ? Elem<T>::load1(row + edge) : __builtin_nanf("");
+#pragma unroll
+        for (int q = 0; q < kVecs; ++q)
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) {
+                if (Tt != 1.0f) v[q][j] = v[q][j] / Tt;
+                if (q * kSmThreads + tid >= nbody) v[q][j] = __builtin_nanf("");
+            }
+        if (Tt != 1.0f) ve = ve / Tt;
+    }
+};
+
+// Part p of row r: the largest key and the sum of exp_det(y - that value) of its elements, left
+// (3 words: key, sum low, sum high) at the start of EVERY part's slice of the row's
+// probabilities, slot p of each.  softmax_write_kernel's workgroup for part q then reads the
+// row's partial results from its own slice before it overwrites it, so the operation needs no
+// workspace and no workgroup waits for another.
+template <typename T>
+__global__ __launch_bounds__(kSmThreads) void softmax_part_kernel(const T* logits, int64_t stride, int V,
+                                                                  int part_len, int nparts,
+                                                                  const float* temperature, float* probs) {
+    constexpr int W = kSmThreads / kWave;
+    __shared__ uint32_t redk[W];
+    __shared__ double redd[W];
+    const int r = blockIdx.x / nparts, p = blockIdx.x - r * nparts;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const float Tt = temperature ? temperature[r] : 1.0f;
+    SoftmaxPart<T> sp;
+    sp.load(logits + (size_t)r * stride, V, part_len, p, Tt);
+    float mx = sp.ve;
+#pragma unroll
+    for (int q = 0; q < SoftmaxPart<T>::kVecs; ++q)
+#pragma unroll
+        for (int j = 0; j < SoftmaxPart<T>::VEC; ++j) mx = __builtin_fmaxf(mx, sp.v[q][j]);  // (NaN ignored)
+    const uint32_t wk = wave_max_u32(key_of(mx));
+    if ((tid & 63) == 0) redk[wave] = wk;
+    __syncthreads();
+    uint32_t mk = 0u;
+#pragma unroll
+    for (int w = 0; w < W; ++w) mk = mk > redk[w] ? mk : redk[w];
+    const float m = mk ? val_of(mk) : -__builtin_inff();
+    // exp_det is 0 for NaN: padding, NaN logits, and y - m of infinities
+    double s = (double)exp_det(sp.ve - m);
+#pragma unroll
+    for (int q = 0; q < SoftmaxPart<T>::kVecs; ++q)
+#pragma unroll
+        for (int j = 0; j < SoftmaxPart<T>::VEC; ++j) s += (double)exp_det(sp.v[q][j] - m);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+    if ((tid & 63) == 0) redd[wave] = s;
+    __syncthreads();
+    if (tid < nparts) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) t += redd[w];
+        const uint64_t b = (uint64_t)__double_as_longlong(t);
+        uint32_t* slot = reinterpret_cast<uint32_t*>(probs + (size_t)r * V + (size_t)tid * part_len) + 3 * p;
+        slot[0] = mk;
+        slot[1] = (uint32_t)b;
+        slot[2] = (uint32_t)(b >> 32);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSmThreads) void softmax_write_kernel(const T* logits, int64_t stride, int V,
+                                                                   int part_len, int nparts,
+                                                                   const float* temperature, float* probs,
+                                                                   float* row_max, float* log_sum) {
+    constexpr int VEC = Elem<T>::kVec;
+    const int r = blockIdx.x / nparts, p = blockIdx.x - r * nparts;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const float Tt = temperature ? temperature[r] : 1.0f;
+    float* out = probs + (size_t)r * V;
+    // every wave combines the row's parts, one per lane (nparts <= 64)
+    const uint32_t* slot = reinterpret_cast<const uint32_t*>(out + (size_t)p * part_len) + 3 * lane;
+    const bool have = lane < nparts;
+    const uint32_t pk = have ? slot[0] : 0u;
+    const uint64_t pb = have ? ((uint64_t)slot[2] << 32) | slot[1] : 0ull;
+    SoftmaxPart<T> sp;
+    sp.load(logits + (size_t)r * stride, V, part_len, p, Tt);
+    const uint32_t mk = wave_max_u32(pk);
+    const float m = mk ? val_of(mk) : -__builtin_inff();  // (a row of NaN: the empty maximum)
+    // a part without a finite maximum adds nothing, and without a finite row maximum S is 0
+    const bool fin = __builtin_fabsf(m) < __builtin_inff() && pk > 0x007FFFFFu;
+    double S = fin ? __longlong_as_double((long long)pb) * exp((double)val_of(pk) - (double)m) : 0.0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) S += __shfl_xor(S, o, kWave);
+    const double inv = 1.0 / S;
+    __syncthreads();  // every wave has read the slots: the slice may be written
+    typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for (int q = 0; q < SoftmaxPart<T>::kVecs; ++q) {
+        const int vi = q * kSmThreads + tid;
+        if (vi >= sp.nbody) break;
+#pragma unroll
+        for (int g = 0; g < VEC / 4; ++g) {
+            F4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = (float)((double)exp_det(sp.v[q][4 * g + j] - m) * inv);
+            *reinterpret_cast<F4*>(out + sp.a + vi * VEC + 4 * g) = o;
+        }
+    }
+    if (sp.edge >= 0) out[sp.edge] = (float)((double)exp_det(sp.ve - m) * inv);
+    if (p == 0 && tid == 0) {
+        if (row_max) row_max[r] = m;
+        if (log_sum) log_sum[r] = (float)log(S);
+    }
+}
+
 // In-place vLLM-v1 penalties on fp32 rows: one workgroup per row, history deduplicated in a
 // per-row hash in the workspace.
 __global__ __launch_bounds__(kOpThreads) void penalties_kernel(KArgs a, float* logits) {
@@ -286,11 +433,17 @@ __global__ void token_state_kernel(uint32_t* st, int64_t stride, uint32_t* bits,
     if (bits) atomicOr(bits + (size_t)rr * (size_t)bstride + ((uint32_t)t >> 5), 1u << (t & 31));
 }
 
-template __global__ void argmax_kernel<float>(const float*, int64_t, int, int32_t*);
-template __global__ void argmax_kernel<uint16_t>(const uint16_t*, int64_t, int, int32_t*);
-template __global__ void softmax_kernel<float>(const float*, int64_t, int, const float*, float*, float*, float*);
-template __global__ void softmax_kernel<uint16_t>(const uint16_t*, int64_t, int, const float*, float*, float*, float*);
-template __global__ void argmax_kernel<_Float16>(const _Float16*, int64_t, int, int32_t*);
-template __global__ void softmax_kernel<_Float16>(const _Float16*, int64_t, int, const float*, float*, float*, float*);
+#define VWS_OPS_INST(T)                                                                             \
+    template __global__ void argmax_kernel<T>(const T*, int64_t, int, int32_t*);                    \
+    template __global__ void softmax_kernel<T>(const T*, int64_t, int, const float*, float*, float*, \
+                                               float*);                                             \
+    template __global__ void softmax_part_kernel<T>(const T*, int64_t, int, int, int, const float*,  \
+                                                    float*);                                        \
+    template __global__ void softmax_write_kernel<T>(const T*, int64_t, int, int, int, const float*, \
+                                                     float*, float*, float*);
+VWS_OPS_INST(float)
+VWS_OPS_INST(uint16_t)
+VWS_OPS_INST(_Float16)
+#undef VWS_OPS_INST
 
 }  // namespace vws

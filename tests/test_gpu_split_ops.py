@@ -54,3 +54,30 @@ def test_softmax_over_its_logits(cuda, V):
     _lib.check(_lib.lib().vws_softmax(x.data_ptr(), _lib.DTYPE_F32, 5, V, V, None, x.data_ptr(), None,
                                       None, torch.cuda.current_stream().cuda_stream))
     torch.testing.assert_close(x, want, rtol=1e-6, atol=1e-12)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["noise", "ties", "constant", "sparse"])
+@pytest.mark.parametrize("B,V,k", [(1, 7, 7), (3, 257, 256), (3, 4097, 1), (16, 128257, 20), (9, 70001, 100),
+                                   (2, 262144, 256), (700, 33000, 40)])
+def test_topk_parts(cuda, dtype, kind, B, V, k):
+    """Row parts, their cut, the merge's cut and the exact selection of rows whose lists overflow
+    (heavy ties), against a stable sort: values and ids exactly."""
+    import torch
+
+    from vllm_webgpu_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(V + k)
+    x = torch.randn((B, V), generator=g, device=cuda) * 3
+    if kind == "ties":
+        x = torch.round(x)
+    elif kind == "constant":
+        x[:] = 1.5
+        x[0, V - 1] = 2.0
+    elif kind == "sparse":
+        x = torch.where(torch.rand((B, V), generator=g, device=cuda) < 0.5 * k / V, x, -float("inf"))
+    x = x.to(torch.float32 if dtype == "f32" else torch.bfloat16)
+    for _ in range(2):  # the counters are left ready for the next call
+        vals, ids = ops.topk(x, k)
+        want, order = torch.sort(x.float(), dim=1, descending=True, stable=True)
+        assert torch.equal(vals, want[:, :k]) and torch.equal(ids.long(), order[:, :k])

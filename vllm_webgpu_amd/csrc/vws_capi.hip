@@ -105,8 +105,10 @@ DeviceInfo device_info() {
 }
 
 // Parts per row for the split-row top-k kernel: enough workgroups to fill every slot of the chip
-// once, with at least 4096 elements per part.
-void choose_parts(int B, int V, int esize, int* S, int* part_len) {
+// once, with at least 4096 elements per part, and few enough that their lists (k entries and
+// some ties each) fit the last part's merge: a row whose lists do not is selected again from the
+// whole row (k = 256, 151936 fp32 in 16 parts 148 us, in 6 parts 49 us).
+void choose_parts(int B, int V, int k, int* S, int* part_len) {
     const DeviceInfo d = device_info();
     const int slots = d.cus * d.fast_blocks_per_cu;
     int s = slots / (B > 0 ? B : 1);
@@ -114,19 +116,18 @@ void choose_parts(int B, int V, int esize, int* S, int* part_len) {
     if (s > kMaxParts) s = kMaxParts;
     const int max_by_len = V / 4096 > 0 ? V / 4096 : 1;
     if (s > max_by_len) s = max_by_len;
+    const int max_by_merge = kMergeCap / (k + k / 8 + 8);
+    if (s > max_by_merge) s = max_by_merge;
     const int min_parts = (V + kPartMax - 1) / kPartMax;  // kMaxParts parts cover VWS_MAX_VOCAB
     if (s < min_parts) s = min_parts;
     int len = (V + s - 1) / s;
     const int align = 64;  // elements; keeps every part start 16-byte aligned
     len = (len + align - 1) / align * align;
     if (len > kPartMax) len = kPartMax;
-    (void)esize;
     s = (V + len - 1) / len;
     *S = s;
     *part_len = len;
 }
-
-int esize_of(int dtype) { return dtype == VWS_DTYPE_F32 ? 4 : 2; }
 
 // Per-device address of `scratch`, looked up once per device with that device current and
 // cleared once by a fill kernel on the caller's stream (the kernels also clear what they use).
@@ -550,7 +551,7 @@ int vws_topk(const void* logits, int32_t dtype, int32_t batch, int32_t vocab, in
     ka.topk_k = k;
     ka.topk_vals = out_vals;
     ka.topk_ids = out_ids;
-    choose_parts(batch, vocab, esize_of(dtype), &ka.S, &ka.part_len);
+    choose_parts(batch, vocab, k, &ka.S, &ka.part_len);
     hipStream_t s = (hipStream_t)stream;
     const int bp = (batch + 7) / 8 * 8;
     const int K = VWS_KERNEL_TOPK;

@@ -995,7 +995,7 @@ __device__ __forceinline__ bool row_tail_small(const KArgs& a, RowSmem& sm, int 
     if (!(m > -__builtin_inff() && m < __builtin_inff())) return false;  // degenerate row
     // fewer candidates than k (no threshold used): every candidate is in the top k
     const uint32_t ykth = total >= k ? (uint32_t)(sm.tk[k - 1] >> 32) : 0u;
-    if (total > kWave && (uint32_t)(sm.tk[kWave] >> 32) >= ykth) return false;  // > 64 tied members
+    if (total > kWave && (uint32_t)(sm.tk[kWave] >> 32) >= ykth) return false;  // > 64 tied members (row_ties)
     auto store_u = [&]() __attribute__((always_inline)) {
         if (sampling && mpos < (uint32_t)kWave) sm.tu[mpos] = u_mine;
     };
@@ -1933,6 +1933,134 @@ __device__ __noinline__ int row_logprobs_entry(int r, uint64_t kernarg) {
 #endif
 }
 
+// A row with k <= 64 whose members tied at the k-th value exceed the 64 slots of row_tail_small,
+// finished from the packed candidates (every thread calls it, after a barrier): one candidate per
+// thread, its cumulative mass counted over all of them, the race reduced over the workgroup.
+// 16-bit logits make such ties common: rows of 262144 soft-capped f16 logits with k = 64 took
+// 610 us on the multi-pass path, 54 us here.  Returns 0 when the row must take that path
+// after all (raw logprobs below the candidates).
+__device__ __noinline__ int row_ties_entry(int r, uint64_t kernarg) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const KArgs a = kargs_at(kernarg);
+    r = __builtin_amdgcn_readfirstlane(r);
+    const RowP prm = row_params(a, r);
+    RowSmem& sm = g_row_sh.f;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int total = (int)sm.npack;
+    const uint32_t ykth = (uint32_t)(sm.tk[prm.k - 1] >> 32);
+    const float m = val_of((uint32_t)(sm.tk[0] >> 32));  // (finite: row_ties has checked)
+    const float lp_min = (prm.min_p > 0.0f) ? log_det(prm.min_p < 1.0f ? prm.min_p : 1.0f)
+                                            : -__builtin_inff();
+    const bool mine = tid < total;
+    const uint64_t key = mine ? sm.pk64[tid] : 0ull;
+    const uint32_t yk = (uint32_t)(key >> 32);
+    const float d = val_of(yk) - m;
+    const bool keep = mine && yk >= ykth && d >= lp_min;
+    const float u = keep ? row_uniform(a, r, (int)(uint32_t)key) : 0.5f;
+    const float e = keep ? exp_det(d) : 0.0f;
+    const uint64_t w = keep ? mass_of(e) : 0ull;
+    // (key, mass) of every candidate, one 16-byte LDS read each, over the buffers (done with)
+    uint4* km = reinterpret_cast<uint4*>(&sm.ckey[0][0]);
+    static_assert(sizeof(sm.ckey) >= kRowPack * sizeof(uint4), "one entry per packed candidate");
+    if (mine) km[tid] = make_uint4((uint32_t)key, yk, (uint32_t)w, (uint32_t)(w >> 32));
+    const uint64_t ww = wave_sum_u64(w);
+    if (lane == 0) sm.red[wave][0] = ww;
+    __syncthreads();
+    uint64_t C = 0ull;
+    const uint64_t W = wave_sum_u64(lane < kRowWaves ? sm.red[lane][0] : 0ull);
+    if (keep) {
+#pragma unroll 4
+        for (int i = 0; i < total; ++i) {
+            const uint4 x = km[i];
+            C += (((uint64_t)x.y << 32) | x.x) <= key ? ((uint64_t)x.w << 32) | x.z : 0ull;
+        }
+    }
+    const float q32 = 1.0f - prm.top_p;
+    const bool topp = q32 > 0.0f;
+    const bool abl = topp && !(q32 < 1.0f);  // top_p <= 0: only the last survivor is kept
+    const uint64_t thr = (topp && !abl) ? scale_floor(q32, W) : 0ull;
+    RowRace rs;
+    if (keep) {
+        if (topp && (abl ? (C != W) : (C <= thr && C != W))) {
+            rs.cprev = C;
+            rs.nrem = 1;
+        } else {
+            rs.cat = C;
+            rs.nkept = 1;
+            rs.last = key;
+            rs.add_key(e / (0.0f - log_det(u)), (int)(uint32_t)key);
+        }
+    }
+    rs.shfl_merge(32); rs.shfl_merge(16); rs.shfl_merge(8);
+    rs.shfl_merge(4); rs.shfl_merge(2); rs.shfl_merge(1);
+    __syncthreads();
+    if (lane == 0) {
+        sm.red[wave][0] = rs.best; sm.red[wave][1] = rs.last; sm.red[wave][2] = rs.cprev;
+        sm.red[wave][3] = rs.cat; sm.red[wave][4] = rs.second;
+        sm.red[wave][5] = ((uint64_t)rs.nrem << 32) | rs.nkept;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        RowRace o;
+        if (lane < kRowWaves) {
+            o.best = sm.red[lane][0]; o.last = sm.red[lane][1]; o.cprev = sm.red[lane][2];
+            o.cat = sm.red[lane][3]; o.second = (uint32_t)sm.red[lane][4];
+            o.nkept = (uint32_t)sm.red[lane][5]; o.nrem = (uint32_t)(sm.red[lane][5] >> 32);
+        }
+        o.shfl_merge(8); o.shfl_merge(4); o.shfl_merge(2); o.shfl_merge(1);
+        rs = o;
+    }
+    if (tid == 0) {
+        uint32_t fl = 0u;
+        // no valid race key: the largest (y, index) kept
+        uint32_t tok = (uint32_t)(rs.best ? 0x7FFFFFFFull - (uint32_t)rs.best : rs.last);
+        if (rs.best && rs.second) {
+            const float bk = u2f((uint32_t)(rs.best >> 32)), sk = u2f(rs.second - 1u);
+            if ((double)sk >= (double)bk * (1.0 - 1e-6)) fl |= VWS_FLAG_RACE_NEAR_TIE;
+        }
+        if (topp && !abl) {
+            const uint64_t tol = (uint64_t)((double)W * 1e-6);
+            if ((rs.nrem > 0u && thr - rs.cprev <= tol) || (rs.cat > thr && rs.cat - thr <= tol))
+                fl |= VWS_FLAG_TOPP_NEAR_TIE;
+        }
+        a.sampled[r] = (int32_t)tok;
+        if (a.flags) a.flags[r] = fl;
+        if (a.nkept) a.nkept[r] = (int32_t)rs.nkept;
+        // for row_logprobs_entry: the token, 64-bit packing, not greedy, the largest threshold
+        // (no wave's is below the seed)
+        sm.lpk[0] = tok; sm.lpk[1] = 1u; sm.lpk[2] = 0u; sm.lpk[3] = sm.tmaxk;
+    }
+    return (a.L < 0 || row_logprobs_entry(r, kernarg)) ? 1 : 0;
+#else
+    (void)r;
+    (void)kernarg;
+    return 0;
+#endif
+}
+
+// Whether row_fast left row r only because more than 64 members tie at its k-th value (k <= 64).
+// Read off the LDS state it leaves, which is its own when it went past its early returns (the
+// conditions repeated here; no top-p path runs for such a row): without a status bit and with
+// 65 to kRowPack candidates packed, row_tail_small ran and filled the 65 slots, and it leaves
+// such a row for a maximum that is not finite or for its ties alone.  A mark written by row_fast,
+// or an argument passed on, moves the row kernel's register allocation (256 masked rows of
+// 128256 fp32 34.7 -> 38 us; 256 rows with 20 logprobs 39 -> 41 us).
+template <typename T>
+__device__ __forceinline__ bool row_ties(const KArgs& a, const RowSmem& sm, int r, const RowP& p) {
+    const bool lp = a.L >= 0;
+    const int k = a.allowed && lp ? fast_k<true>(a, p) : fast_k<false>(a, p);
+    if (a.nofast || p.greedy || k == 0 || k > kWave || (lp && a.softcap > 0.0f)) return false;
+    Slice<T> sl;
+    sl.init(reinterpret_cast<const T*>(a.logits) + (size_t)r * a.lstride, 0, a.V);
+    if (a.allowed && !lp && sl.a != 0) return false;
+    if (p.tab && !(p.rep >= 1.0f && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
+    const uint32_t n = tp_u(sm.npack);
+    if (tp_u(sm.status) != 0u || n <= (uint32_t)kWave || n > (uint32_t)kRowPack) return false;
+    const uint32_t y0 = tp_u((uint32_t)(sm.tk[0] >> 32));
+    return y0 > 0x007FFFFFu && y0 < 0xFF800000u &&
+           tp_u((uint32_t)(sm.tk[kWave] >> 32)) >= tp_u((uint32_t)(sm.tk[k - 1] >> 32));
+}
+
 // The general path runs in a function of its own so that its register allocation (it needs
 // more than the 128 VGPRs a 1024-thread workgroup allows and spills) stays out of the
 // single-pass loop.  The kernel hands it the address of its kernarg segment (a callee has no
@@ -1943,6 +2071,30 @@ __device__ __noinline__ void row_general(int r, uint64_t kernarg) {
     const KArgs a = kargs_at(kernarg);
     const RowP prm = row_params(a, r);
     general_row<T>(a, g_row_sh.g, r, prm);
+#else
+    (void)r;
+    (void)kernarg;
+#endif
+}
+
+// A row that neither single pass finished: from its candidates when only its ties kept the single
+// pass from finishing it, else on the multi-pass path.  A function in front of the two, so that
+// the row kernel makes one call, as it did without the ties, and a row with ties does not pay
+// the multi-pass path's saved registers.
+template <typename T>
+__device__ __noinline__ void row_rest(int r, uint64_t kernarg) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    bool ties;
+    {
+        const KArgs a = kargs_at(kernarg);
+        const int rr = __builtin_amdgcn_readfirstlane(r);
+        ties = row_ties<T>(a, g_row_sh.f, rr, row_params(a, rr));
+    }
+    if (ties) {
+        if (row_ties_entry(r, kernarg)) return;
+        __syncthreads();
+    }
+    row_general<T>(r, kernarg);
 #else
     (void)r;
     (void)kernarg;
@@ -2011,7 +2163,7 @@ __device__ __forceinline__ bool row_one(const KArgs& a, int r, const void* logit
         if (why == 0) return true;
     }
     __syncthreads();
-    row_general<T>(r, kernarg);
+    row_rest<T>(r, kernarg);
     // diagnostic: why the single-pass top-p path handed the row over (thread 0 wrote the flags)
     if (why && threadIdx.x == 0 && a.flags) a.flags[r] |= (uint32_t)why << 16;
     return true;

@@ -1,0 +1,120 @@
+"""Launches whose rows nothing cuts (temperature alone): the split single-read kernel against the
+oracle and against the multi-pass path (the single passes switched off), which must agree exactly
+in tokens, flags and survivor counts."""
+import numpy as np
+import pytest
+
+from oracle import sampler as O
+
+pytestmark = pytest.mark.gpu
+
+DT = ("f32", "bf16", "f16")
+
+
+def _run(x, T, both=True, **kw):
+    """The launch on the plain kernel and, with the single passes off, on the multi-pass path."""
+    import torch
+
+    from vllm_webgpu_amd import _lib, ops
+
+    L = _lib.lib()
+    out = []
+    for on in ((1, 0) if both else (1,)):
+        before = L.vws_set_single_pass(on)
+        try:
+            r = ops.sample(x, temperature=T, **kw)
+            torch.cuda.synchronize()
+        finally:
+            L.vws_set_single_pass(before)
+        out.append((r.sampled.cpu().numpy(), r.flags.cpu().numpy().view(np.uint32), r.num_kept.cpu().numpy()))
+    return out
+
+
+def _same(a, b):
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1] & 0xFF, b[1] & 0xFF) and np.array_equal(a[2], b[2])
+
+
+def _logits(cuda, B, V, dtype, scale=3.0, seed=0):
+    import torch
+
+    g = torch.Generator(device=cuda).manual_seed(seed * 31 + V)
+    x = torch.randn((B, V), generator=g, device=cuda) * scale
+    return x.to({"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]), g
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("B,V", [(3, 1), (3, 3), (5, 7), (4, 2047), (3, 8193), (17, 50257), (130, 32001),
+                                 (2, 524288), (2100, 1003)])
+def test_plain_rows(cuda, dtype, given, B, V):
+    """Block and part edges, odd rows of 16-bit logits, one part per row (B > 2048), greedy rows
+    among the others, temperatures from 0.02 to 50."""
+    import torch
+
+    x, g = _logits(cuda, B, V, dtype)
+    T = torch.exp(torch.linspace(-3.9, 3.9, B, device=cuda))
+    T[1::5] = 0.0
+    if given:
+        kw = {"uniforms": torch.randint(0, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24}
+    else:
+        kw = {"rng_seeds": torch.arange(B, device=cuda) * 977 + V, "rng_offsets": torch.arange(B, device=cuda) << 33}
+    fast, slow = _run(x, T, **kw)
+    assert not (fast[1] & 0x100).any() and (slow[1] & 0x100).all()
+    _same(fast, slow)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("kind", ["constant", "rounded", "neg_inf", "nan", "inf", "peaked", "ascending", "tiny_T"])
+def test_plain_values(cuda, dtype, kind):
+    """Rows the short lists cannot decide (equal keys, no finite maximum) and values that reach
+    none of the bounds' comparisons."""
+    import torch
+
+    B, V = 6, 40003
+    x, g = _logits(cuda, B, V, dtype, seed=1)
+    T = torch.full((B,), 0.9, device=cuda)
+    kw = {"rng_key": 12345}
+    if kind == "constant":
+        x[:] = 1.25
+        x[0] = -float("inf")
+        kw = {"uniforms": torch.full((B, V), 0.75, device=cuda)}
+        kw["uniforms"][2, 17] = kw["uniforms"][2, 30000] = 0.875
+        kw["uniforms"][3] = 0.0
+    elif kind == "rounded":
+        x = torch.round(x)
+        kw = {"uniforms": torch.randint(1, 64, (B, V), generator=g, device=cuda).float() / 64}
+    elif kind == "neg_inf":
+        x[:, : V - 9] = -float("inf")
+        x[1, 1:] = -float("inf")
+    elif kind == "nan":
+        x[:, ::3] = float("nan")
+        x[1] = float("nan")
+    elif kind == "inf":
+        x[0, 5] = x[0, 9] = float("inf")
+        x[1, 7] = float("inf")
+        x[1, 3] = float("nan")
+    elif kind == "peaked":
+        x[:, 123] = 60.0
+    elif kind == "ascending":
+        x = torch.sort(x, dim=1).values
+    else:
+        T[:] = 2e-5
+    _same(*_run(x, T, **kw))
+
+
+def test_plain_oracle(cuda):
+    """Full-size rows against the sequential oracle (given uniforms), the whole batch twice (the
+    arrival counters are left ready)."""
+    import torch
+
+    B, V = 24, 128256
+    x, g = _logits(cuda, B, V, "f32", seed=2)
+    u = torch.randint(1, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24
+    T = np.linspace(0.3, 1.5, B).astype(np.float32)
+    one = np.ones(B, np.float32)
+    ref = O.sample(x.cpu().numpy(), O.make_params(B, T, np.zeros(B, np.int32), one, 0 * one, one, 0 * one, 0 * one),
+                   u.cpu().numpy())
+    for _ in range(2):
+        got, = _run(x, torch.from_numpy(T).to(cuda), both=False, uniforms=u)
+        assert np.array_equal(got[0], ref["token"]) and np.array_equal(got[1] & 0xFF, ref["flags"] & 0xFF)
+        assert np.array_equal(got[2], ref["n_kept"])

@@ -11,12 +11,14 @@
 #include <string>
 
 #include "vws_internal.h"
+#include "vws_plain.h"
 #include "vws_sampler.h"
 
 namespace vws {
 template <typename T> __global__ void fast_kernel(KArgs);
 template <typename T> __global__ void general_kernel(KArgs);
 template <typename T, bool LP, int XF> __global__ void row_kernel(const void*, int64_t, int, int, KArgs);
+template <typename T> __global__ void plain_kernel(PlainArgs);
 template <typename T> __global__ void argmax_kernel(const T*, int64_t, int, int32_t*);
 template <typename T>
 __global__ void softmax_kernel(const T*, int64_t, int, const float*, float*, float*, float*);
@@ -36,7 +38,11 @@ using namespace vws;
 // Static device scratch of vws_sample_noalloc (one copy per GPU, held until the process ends).
 // Host code never uses this name as an address: the per-device address comes from
 // hipGetSymbolAddress (scratch_address below) and only that pointer is handed to kernels.
-static __device__ __align__(256) unsigned char scratch[VWS_NOALLOC_SCRATCH_BYTES];
+// The plain rows' records come on top of the documented size, so that they leave the accepted
+// batches as they are.
+constexpr size_t kPlainBytes = sizeof(CoopState::plain_ctr) + sizeof(CoopState::plain_rec);
+constexpr size_t kScratchBytes = VWS_NOALLOC_SCRATCH_BYTES + kPlainBytes;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 
@@ -157,7 +163,7 @@ int scratch_address(hipStream_t s, void** out) {
         if (hipStreamIsCapturing(s, &cs) != hipSuccess) cs = hipStreamCaptureStatusNone;
         (void)hipGetLastError();
         if (cs == hipStreamCaptureStatusNone) {
-            const size_t n = VWS_NOALLOC_SCRATCH_BYTES / 4;
+            const size_t n = kScratchBytes / 4;
             hipLaunchKernelGGL(fill_u32_kernel, dim3(1024), dim3(256), 0, s, static_cast<uint32_t*>(p), n, 0u);
             if (int st = check_launch("vws_sample_noalloc (scratch clear)")) return st;
             const hipError_t se = hipStreamSynchronize(s);
@@ -307,6 +313,60 @@ KArgs make_kargs(int B, int V, const void* logits, int64_t stride, void* ws, int
     return k;
 }
 
+// Whether nothing cuts, changes or reports on the launch's rows but the temperature: no top-k,
+// top-p or min-p arrays, no history, processors, mask or soft cap, no logprobs (the sampling
+// defaults: every request's parameters off).  Known without reading the parameters; a launch with
+// such rows among others takes the row kernel.
+bool plain_launch(const vws_sample_args* a) {
+    return a->temperature && !a->top_k && !a->top_p && !a->min_p && !a->prompt_ids && !a->output_ids &&
+           !a->adjust_ids && !a->token_state && !a->allowed_mask && !(a->logit_softcap > 0.0f) &&
+           a->num_logprobs < 0 && g_single_pass.load(std::memory_order_relaxed);
+}
+
+int sample_plain(const vws_sample_args* a, void* ws) {
+    PlainArgs k;
+    std::memset(&k, 0, sizeof(k));
+    k.logits = a->logits;
+    k.lstride = a->logits_row_stride;
+    k.V = a->vocab;
+    k.temperature = a->temperature;
+    k.u = a->uniforms;
+    k.ustride = a->uniforms_row_stride;
+    k.rng_seed = a->uniforms ? nullptr : a->rng_seeds;
+    k.rng_offset = a->uniforms ? nullptr : a->rng_offsets;
+    k.rng_key = a->rng_key;
+    k.sampled = a->sampled;
+    k.flags = a->row_flags;
+    k.nkept = a->num_kept;
+    // parts of at least 4096 tokens, four workgroups (of four waves) for each compute unit: one
+    // round of the chip (128 x 151936 bf16: 3 / 4 / 5 / 7 / 8 workgroups 35.1 / 33.5 / 32.9 / 36.2 /
+    // 39.3 us; 256 x 151936 fp32 with given uniforms 62.6 / 56.1 / 56.7 / 71.0 / 70.9 us); one part per
+    // row without the workspace or when the rows exceed its records
+    int s = 1;
+    if (ws) {
+        const int B = a->batch;
+        s = 4 * device_info().cus / B;
+        if (s > kPlRecs / B) s = kPlRecs / B;
+        if (s > a->vocab / 4096) s = a->vocab / 4096;
+        if (s > kPlMaxParts) s = kPlMaxParts;
+        if (s < 1) s = 1;
+        CoopState* st = static_cast<CoopState*>(ws);  // (first in the workspace)
+        k.rec = st->plain_rec;
+        k.ctr = st->plain_ctr;
+    }
+    const int nblk = a->vocab / 4;
+    k.part_blocks = (nblk + s - 1) / s;
+    k.S = k.part_blocks > 0 ? (nblk + k.part_blocks - 1) / k.part_blocks : 1;
+    hipStream_t st = (hipStream_t)a->stream;
+    const int K = VWS_KERNEL_SAMPLE;
+    const dim3 grid((unsigned)a->batch * (unsigned)k.S), block(kPlThreads);
+    if (a->dtype == VWS_DTYPE_F32) launch(K, plain_kernel<float>, grid, block, st, k);
+    else if (a->dtype == VWS_DTYPE_BF16) launch(K, plain_kernel<uint16_t>, grid, block, st, k);
+    else launch(K, plain_kernel<_Float16>, grid, block, st, k);
+    if (int rc = check_launch("vws_sample (plain rows)")) return rc;
+    return ok();
+}
+
 // Rows of up to kSmRowMax elements take one workgroup each, longer ones parts of at most
 // kSmPartMax: two launches, but every compute unit at work and no thread with more than 32
 // elements.  Measured, one workgroup per row against parts (fp32, a call): 1 x 5000 13.4 and
@@ -367,6 +427,7 @@ int vws_sample(const vws_sample_args* a) {
     int st = validate_sample(a);
     if (st) return st;
     const int hw = sample_history_width(a);
+    if (plain_launch(a)) return sample_plain(a, sample_workspace(a, hw));
     KArgs k = make_kargs(a->batch, a->vocab, a->logits, a->logits_row_stride, sample_workspace(a, hw), hw, false);
     k.temperature = a->temperature;
     k.top_k = a->top_k;
@@ -470,18 +531,18 @@ int vws_sample_noalloc(const vws_sample_args* a) {
     const int hw = sample_history_width(a);
     if (hw < 0) return validate_sample(a);
     const size_t need = ws_layout(a->batch, a->vocab, hw, false).total;
-    if (need > (size_t)VWS_NOALLOC_SCRATCH_BYTES)
+    if (need > kScratchBytes)
         return fail(VWS_ERR_LIMIT,
                     "vws_sample_noalloc: this batch needs %zu bytes of scratch (batch %d, history width %d); "
                     "the static scratch holds %zu (use vws_sample with a caller workspace)",
-                    need, a->batch, hw, (size_t)VWS_NOALLOC_SCRATCH_BYTES);
+                    need, a->batch, hw, kScratchBytes);
     vws_sample_args b = *a;
     b.workspace = nullptr;
     b.workspace_bytes = 0;
     if (need) {
         // arguments first (host only), so a bad call touches no device state
         b.workspace = reinterpret_cast<void*>(uintptr_t(256));
-        b.workspace_bytes = VWS_NOALLOC_SCRATCH_BYTES;
+        b.workspace_bytes = kScratchBytes;
         if (int st = validate_sample(&b)) return st;
         void* p = nullptr;
         if (int st = scratch_address((hipStream_t)a->stream, &p)) return st;

@@ -19,6 +19,12 @@ constexpr int kMergeCap = kFastWaves * kCapW;     // entries the last part can m
 constexpr int kPartMax = 32768;                   // elements per part
 constexpr int kMaxParts = 16;                    // parts per row: VWS_MAX_VOCAB / kPartMax
 
+// Plain rows (vws_plain.hip): threads per part, most parts of a row, and the records of a launch
+// (parts of all its rows) the workspace holds.
+constexpr int kPlThreads = 256;
+constexpr int kPlMaxParts = 32;
+constexpr int kPlRecs = 2048;
+
 // Split softmax (vws_ops.hip): threads per part, most elements of a part (32 per thread, kept in
 // registers) and most parts of a row (VWS_MAX_VOCAB / kSmPartMax; one lane of a wave each).
 constexpr int kSmThreads = 256;
@@ -96,6 +102,9 @@ struct CoopState {
     uint64_t wgs;
     uint32_t pad[62];
     CoopSlot slot[kCoopSlots];
+    // plain rows split over several workgroups: parts arrived per row (left at zero) and records
+    uint32_t plain_ctr[kPlRecs];
+    uint64_t plain_rec[(size_t)kPlRecs * 8];
 };
 
 struct KArgs {

@@ -64,7 +64,8 @@ def test_plain_rows(cuda, dtype, given, B, V):
 
 
 @pytest.mark.parametrize("dtype", DT)
-@pytest.mark.parametrize("kind", ["constant", "rounded", "neg_inf", "nan", "inf", "peaked", "ascending", "tiny_T"])
+@pytest.mark.parametrize("kind", ["constant", "rounded", "neg_inf", "nan", "inf", "peaked", "ascending", "tiny_T",
+                                  "lost_peak", "huge"])
 def test_plain_values(cuda, dtype, kind):
     """Rows the short lists cannot decide (equal keys, no finite maximum) and values that reach
     none of the bounds' comparisons."""
@@ -95,6 +96,17 @@ def test_plain_values(cuda, dtype, kind):
         x[1, 3] = float("nan")
     elif kind == "peaked":
         x[:, 123] = 60.0
+    elif kind == "lost_peak":
+        # u = 0 takes the peak out of the race; the other exponentials are small, subnormal or 0
+        x[:, 123] = torch.linspace(60.0, 115.0, B, device=cuda).to(x.dtype)
+        kw = {"uniforms": torch.randint(1, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24}
+        kw["uniforms"][:, 123] = 0.0
+    elif kind == "huge":
+        # finite logits whose log2(e) / T multiple is not
+        top = torch.finfo(x.dtype).max
+        x = x * (top / 64)
+        x[:, 100], x[:, 39000] = 0.98 * top, 0.6 * top
+        T[:] = 1.0
     elif kind == "ascending":
         x = torch.sort(x, dim=1).values
     else:

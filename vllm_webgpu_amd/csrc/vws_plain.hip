@@ -8,7 +8,8 @@
 // largest seen (a handful), delta a bound on the rounding of both forms, and the part that
 // arrives last computes the exact keys of those alone, with the row maximum known.  A row takes
 // the multi-pass sampler's two passes of exact keys (exact_row) only when the short lists cannot
-// decide it (no finite maximum, uniforms outside [0, 1), more near-equal keys than a list holds).
+// decide it (no finite maximum, uniforms outside [0, 1), more near-equal keys than a list holds, a
+// best key near underflow).
 //
 // Bound: VALU, by the generated uniforms (Philox-4x32-10: 20 quarter-rate 32 x 32 multiplies per
 // four tokens).  E >= 1 - u >= 2^-24 gives each block of four tokens the bound max x c + 24, so
@@ -436,11 +437,15 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
         rr.add_key(exp_det(y - m) / (0.0f - log_det(plain_uniform(a, r, t))), t);
     }
     plain_merge(sm, rr);
-    if (tid == 0) sm.last = rr.best ? 1u : 0u;
-    if (tid == 0 && rr.best)
+    // A key below 2^-100 decides nothing: E >= 2^-24, so its e may be rounded as a subnormal or be
+    // 0 (the largest logits drew u = 0, or a part's x c overflowed and its list is empty), and the
+    // order of g is not the keys' there.
+    const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-100f;
+    if (tid == 0) sm.last = won ? 1u : 0u;
+    if (tid == 0 && won)
         plain_write(a, r, (int32_t)(0x7FFFFFFF - (uint32_t)rr.best), plain_near_tie(rr), (int32_t)count);
     __syncthreads();
-    if (!sm.last) exact_row<T>(a, sm, r, row, Tt, maxk);  // no valid key among them
+    if (!sm.last) exact_row<T>(a, sm, r, row, Tt, maxk);
 }
 
 template __global__ void plain_kernel<float>(PlainArgs);

@@ -130,3 +130,31 @@ def test_plain_oracle(cuda):
         got, = _run(x, torch.from_numpy(T).to(cuda), both=False, uniforms=u)
         assert np.array_equal(got[0], ref["token"]) and np.array_equal(got[1] & 0xFF, ref["flags"] & 0xFF)
         assert np.array_equal(got[2], ref["n_kept"])
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("B,V", [(1, 4095), (1, 8192), (3, 8193), (7, 40003), (1, 524288), (128, 9001), (129, 9001),
+                                 (256, 9001), (257, 9001), (512, 8191), (513, 8191)])
+def test_greedy_launches(cuda, dtype, B, V):
+    """Launches without temperatures, the rows split or (short rows, many rows) whole: ties within
+    and across parts, zeros of both signs, infinities and NaN; top-k and top-p arrays do not count."""
+    import torch
+
+    x, g = _logits(cuda, B, V, dtype, seed=3)
+    x[0, V // 2 :: 977] = 50.0
+    if B > 2:
+        x[1] = -float("inf")
+        x[1, V - 1] = float("nan")
+        x[2] = -1.0
+        x[2, 5], x[2, V - 2] = -0.0, 0.0
+    if B > 6:
+        x[3] = float("nan")
+        x[4, V - 1] = x[4, V - 3] = float("inf")
+        x[5, ::2] = float("nan")
+        x[5, V - 4 :] = 99.0
+    k = torch.full((B,), 3, dtype=torch.int32, device=cuda)
+    fast, slow = _run(x, None, top_k=k, top_p=k * 0.25)
+    _same(fast, slow)
+    f = x.float().nan_to_num(nan=-float("inf"), posinf=float("inf"), neginf=-float("inf")).cpu().numpy()
+    ok = np.isfinite(f).any(1) | (f == np.inf).any(1)
+    assert np.array_equal(fast[0][ok], f.argmax(1)[ok])

@@ -314,16 +314,30 @@ KArgs make_kargs(int B, int V, const void* logits, int64_t stride, void* ws, int
 }
 
 // Whether nothing cuts, changes or reports on the launch's rows but the temperature: no top-k,
-// top-p or min-p arrays, no history, processors, mask or soft cap, no logprobs (the sampling
-// defaults: every request's parameters off).  Known without reading the parameters; a launch with
-// such rows among others takes the row kernel.
+// top-p or min-p arrays (which a launch without temperatures, all greedy, does not read), no
+// history, processors, mask or soft cap, no logprobs (the sampling defaults: every request's
+// parameters off).  Known without reading the parameters; a launch with such rows among others
+// takes the row kernel.
 bool plain_launch(const vws_sample_args* a) {
-    return a->temperature && !a->top_k && !a->top_p && !a->min_p && !a->prompt_ids && !a->output_ids &&
+    return (!a->temperature || (!a->top_k && !a->top_p && !a->min_p)) && !a->prompt_ids && !a->output_ids &&
            !a->adjust_ids && !a->token_state && !a->allowed_mask && !(a->logit_softcap > 0.0f) &&
            a->num_logprobs < 0 && g_single_pass.load(std::memory_order_relaxed);
 }
 
-int sample_plain(const vws_sample_args* a, void* ws) {
+// Parts per plain row: of at least 4096 tokens, four workgroups (of four waves) for each compute
+// unit: one round of the chip (128 x 151936 bf16: 3 / 4 / 5 / 7 / 8 workgroups 35.1 / 33.5 / 32.9 /
+// 36.2 / 39.3 us; 256 x 151936 fp32 with given uniforms 62.6 / 56.1 / 56.7 / 71.0 / 70.9 us); one
+// part per row without the workspace or when the rows exceed its records.
+int plain_parts(const vws_sample_args* a, const void* ws) {
+    if (!ws) return 1;
+    int s = 4 * device_info().cus / a->batch;
+    if (s > kPlRecs / a->batch) s = kPlRecs / a->batch;
+    if (s > a->vocab / 4096) s = a->vocab / 4096;
+    if (s > kPlMaxParts) s = kPlMaxParts;
+    return s < 1 ? 1 : s;
+}
+
+int sample_plain(const vws_sample_args* a, void* ws, int s) {
     PlainArgs k;
     std::memset(&k, 0, sizeof(k));
     k.logits = a->logits;
@@ -338,18 +352,7 @@ int sample_plain(const vws_sample_args* a, void* ws) {
     k.sampled = a->sampled;
     k.flags = a->row_flags;
     k.nkept = a->num_kept;
-    // parts of at least 4096 tokens, four workgroups (of four waves) for each compute unit: one
-    // round of the chip (128 x 151936 bf16: 3 / 4 / 5 / 7 / 8 workgroups 35.1 / 33.5 / 32.9 / 36.2 /
-    // 39.3 us; 256 x 151936 fp32 with given uniforms 62.6 / 56.1 / 56.7 / 71.0 / 70.9 us); one part per
-    // row without the workspace or when the rows exceed its records
-    int s = 1;
     if (ws) {
-        const int B = a->batch;
-        s = 4 * device_info().cus / B;
-        if (s > kPlRecs / B) s = kPlRecs / B;
-        if (s > a->vocab / 4096) s = a->vocab / 4096;
-        if (s > kPlMaxParts) s = kPlMaxParts;
-        if (s < 1) s = 1;
         CoopState* st = static_cast<CoopState*>(ws);  // (first in the workspace)
         k.rec = st->plain_rec;
         k.ctr = st->plain_ctr;
@@ -427,7 +430,18 @@ int vws_sample(const vws_sample_args* a) {
     int st = validate_sample(a);
     if (st) return st;
     const int hw = sample_history_width(a);
-    if (plain_launch(a)) return sample_plain(a, sample_workspace(a, hw));
+    if (plain_launch(a)) {
+        void* ws = sample_workspace(a, hw);
+        const int s = plain_parts(a, ws);
+        // All-greedy launches: the row kernel gives each row 1024 threads and one compute unit, so
+        // it stays for more than half the compute units' number of rows up to that number (one
+        // nearly full round: 256 x 128256 fp32 / bf16 26.1 / 18.5 us, here 27.7 / 21.2) and for few
+        // rows that are not split.  Otherwise (row kernel, here): 1 x 262144 bf16 17.7, 12.8 us;
+        // 128 x 151936 bf16 17.0, 16.3; 270 x 151936 fp32 56, 32.7; 400 x 32000 fp32 35, 15.3;
+        // 1000 x 6001 fp32 62, 12.8; 1024 x 128256 fp32 118, 81.
+        const int cus = device_info().cus, B = a->batch;
+        if (a->temperature || B > 2 * cus || (s > 1 && (B <= cus / 2 || B > cus))) return sample_plain(a, ws, s);
+    }
     KArgs k = make_kargs(a->batch, a->vocab, a->logits, a->logits_row_stride, sample_workspace(a, hw), hw, false);
     k.temperature = a->temperature;
     k.top_k = a->top_k;

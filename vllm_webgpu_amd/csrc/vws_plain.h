@@ -11,7 +11,7 @@ struct PlainArgs {
     const void* logits;
     int64_t lstride;
     int V;
-    const float* temperature;
+    const float* temperature;    // null: every row greedy
     const float* u;              // [B, V] uniforms, or null: generated
     int64_t ustride;
     const uint64_t* rng_seed;

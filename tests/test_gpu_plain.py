@@ -158,3 +158,33 @@ def test_greedy_launches(cuda, dtype, B, V):
     f = x.float().nan_to_num(nan=-float("inf"), posinf=float("inf"), neginf=-float("inf")).cpu().numpy()
     ok = np.isfinite(f).any(1) | (f == np.inf).any(1)
     assert np.array_equal(fast[0][ok], f.argmax(1)[ok])
+
+
+def test_streams_apart(cuda):
+    """Split rows of launches on several streams without an order between them: each stream has
+    its own workspace, so no launch counts another's parts."""
+    import torch
+
+    from vllm_webgpu_amd import ops
+
+    B, V, n = 24, 40003, 3
+    xs = [_logits(cuda, B, V, "bf16", seed=4 + i)[0] for i in range(n)]
+    T = torch.full((B,), 0.9, device=cuda)
+    calls = [{}, {"temperature": T, "rng_key": 7}]
+    want = [[ops.sample(x, **kw).sampled.cpu() for kw in calls] for x in xs]
+    streams = [torch.cuda.Stream() for _ in range(n)]
+    torch.cuda.synchronize()
+    got = [[] for _ in range(n)]
+    for _ in range(20):
+        for s, x, g in zip(streams, xs, got):
+            with torch.cuda.stream(s):
+                g.extend(ops.sample(x, **kw).sampled for kw in calls)
+    torch.cuda.synchronize()
+    buffers = set()
+    for s in streams:
+        with torch.cuda.stream(s):
+            buffers.add(ops.workspace(1, torch.device("cuda", torch.cuda.current_device())).data_ptr())
+    assert len(buffers) == n
+    for w, g in zip(want, got):
+        for i, t in enumerate(g):
+            assert torch.equal(t.cpu(), w[i % 2])

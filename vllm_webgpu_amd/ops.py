@@ -20,7 +20,9 @@ import torch
 from . import _lib
 
 _ws_lock = threading.Lock()
-_ws_cache: dict[int, torch.Tensor] = {}
+_ws_cache: dict[int, torch.Tensor] = {}               # by device
+_ws_side: dict[tuple[int, int], torch.Tensor] = {}    # by device and stream, other than the default stream
+_WS_SIDE_MAX = 32
 
 
 def _stream_ptr() -> int:
@@ -72,19 +74,40 @@ def _history(ids, lens, B: int, device, name: str):
     return ids, ids.stride(0), ids.shape[1], lens
 
 
-def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
-    """Per-device scratch buffer, grown on demand and cleared once on the current stream.
+def _new_workspace(nbytes: int, idx: int) -> torch.Tensor:
+    ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=f"cuda:{idx}")
+    _lib.check(_lib.lib().vws_workspace_init(ws.data_ptr(), ws.numel(), _stream_ptr()))
+    return ws
 
-    Calls that share a device share this buffer: run them in stream order (one stream), as the
-    sampler kernels leave it clean for the next call but do not guard concurrent use.
+
+def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
+    """Scratch buffer of the device and its current stream, grown on demand and cleared once on
+    that stream.
+
+    The kernels leave the buffer clean for the next call but do not guard concurrent use (the
+    parts of a split row count their arrivals there), so calls that may overlap need buffers of
+    their own: each stream has one, up to ``_WS_SIDE_MAX`` streams besides the default one; calls
+    on further streams, and calls under graph capture on a stream without one, share the device's
+    and must run in stream order with its other users.
     """
     idx = device.index if device.index is not None else torch.cuda.current_device()
+    stream = torch._C._cuda_getCurrentRawStream(idx)
     with _ws_lock:
+        if stream:
+            ws = _ws_side.get((idx, stream))
+            if ws is not None and ws.numel() >= nbytes:
+                return ws
+            if not torch.cuda.is_current_stream_capturing():
+                if ws is not None or len(_ws_side) < _WS_SIDE_MAX:
+                    ws = _ws_side[idx, stream] = _new_workspace(nbytes, idx)
+                    return ws
         ws = _ws_cache.get(idx)
         if ws is None or ws.numel() < nbytes:
-            ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=f"cuda:{idx}")
-            _lib.check(_lib.lib().vws_workspace_init(ws.data_ptr(), ws.numel(), _stream_ptr()))
-            _ws_cache[idx] = ws
+            if stream:  # one that a warm-up on another stream has made, rather than a new one
+                for (i, _), w in _ws_side.items():
+                    if i == idx and w.numel() >= nbytes:
+                        return w
+            ws = _ws_cache[idx] = _new_workspace(nbytes, idx)
         return ws
 
 

@@ -125,7 +125,8 @@ class PreparedSample:
     """One ``vws_sample`` call with its arguments validated and packed once (``prepare_sample``):
     ``launch()`` issues it again on the current stream with one C call, reading the same input
     tensors (their current contents) and writing the same ``result`` tensors.  The object keeps
-    every tensor it points at alive."""
+    every tensor it points at alive, the workspace of the stream it was prepared on among them:
+    launches on another stream must be in order with that stream's calls."""
 
     def __init__(self, args, result: SampleResult, keep: tuple):
         self.args = args

@@ -114,6 +114,37 @@ def test_plain_values(cuda, dtype, kind):
     _same(*_run(x, T, **kw))
 
 
+def _oracle(x, T, u):
+    B = x.shape[0]
+    one = np.ones(B, np.float32)
+    ref = O.sample(x, O.make_params(B, np.full(B, T, np.float32), np.zeros(B, np.int32), one, 0 * one, one, 0 * one,
+                                    0 * one), u)
+    return ref["token"], ref["flags"], ref["n_kept"]
+
+
+@pytest.mark.parametrize("dtype", DT)
+def test_peak_lost_to_a_zero_exponential(cuda, dtype):
+    """Regression: u = 0 takes the peak (token 10) out of the race, and token 100, whose exponential
+    is 0 (81 below the peak), has the largest approximate key of its part, above token 200's, the
+    row's winner.  Another part's 9000 must not win in its place: its key, 2^-94, is small enough
+    for a zero exponential to have hidden a better one."""
+    import torch
+
+    B, V = 2, 16384
+    rng = np.random.default_rng(8)
+    x = rng.normal(-200, 3, (B, V)).astype(np.float32)
+    u = (rng.integers(1, 1 << 24, (B, V)) * 2.0 ** -24).astype(np.float32)
+    for t, v, w in ((10, 0.0, 0.0), (100, -81.0, 1 - 2.0 ** -24), (200, -79.0, 1 - 12 * 2.0 ** -24),
+                    (9000, -79.0, 1 - 16 * 2.0 ** -24)):
+        x[:, t], u[:, t] = v, w
+    ref = _oracle(x, 1.0, u)
+    assert (ref[0] == 200).all()
+    xd, _ = _logits(cuda, B, V, dtype)
+    xd.copy_(torch.from_numpy(x))
+    for got in _run(xd, torch.ones(B, device=cuda), uniforms=torch.from_numpy(u).to(cuda)):
+        _same(got, ref)
+
+
 def test_plain_oracle(cuda):
     """Full-size rows against the sequential oracle (given uniforms), the whole batch twice (the
     arrival counters are left ready)."""

@@ -439,10 +439,11 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
         rr.add_key(exp_det(y - m) / (0.0f - log_det(plain_uniform(a, r, t))), t);
     }
     plain_merge(sm, rr);
-    // A key below 2^-100 decides nothing: E >= 2^-24, so its e may be rounded as a subnormal or be
-    // 0 (the largest logits drew u = 0, or a part's x c overflowed and its list is empty), and the
-    // order of g is not the keys' there.
-    const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-100f;
+    // A key below 2^-91 decides nothing: exp_det is 0 below -80, so an element whose exact key is 0
+    // can have g only 80 log2(e) - 24 = 91.4 below the row maximum's x c (E >= 2^-24), and hide a
+    // better live one of its part (the largest logits drew u = 0, or a part's x c overflowed and
+    // its list is empty).  From 2^-91 on no exponential in reach is 0 and g orders the keys.
+    const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-91f;
     if (tid == 0) sm.last = won ? 1u : 0u;
     if (tid == 0 && won)
         plain_write(a, r, (int32_t)(0x7FFFFFFF - (uint32_t)rr.best), plain_near_tie(rr), (int32_t)count);

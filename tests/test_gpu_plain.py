@@ -145,6 +145,31 @@ def test_peak_lost_to_a_zero_exponential(cuda, dtype):
         _same(got, ref)
 
 
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_scaled_logits_at_the_edge_of_their_range(cuda, sign):
+    """Regression: two neighbouring floats with the same x / T, of which only the one nearer 0 has a
+    finite x log2(e) / T, as the largest of a row (positive, or negative above a mask of the
+    lowest value).  The token with the infinite product races with the smaller exponential
+    variate and wins, whatever the other one's part lists."""
+    import torch
+
+    T, lo, hi = (float.fromhex(v) for v in ("0x1.4ccccc0p+0", "0x1.cd5bd6p+127", "0x1.cd5bd8p+127"))
+    assert np.float32(lo) / np.float32(T) == np.float32(hi) / np.float32(T)
+    B, V = 2, 16384
+    rng = np.random.default_rng(9)
+    x = rng.normal(0, 3, (B, V)).astype(np.float32)
+    if sign < 0:
+        x[:] = np.finfo(np.float32).min
+    u = (rng.integers(1, 1 << 24, (B, V)) * 2.0 ** -24).astype(np.float32)
+    x[:, 10], u[:, 10] = sign * hi, 0.75
+    x[:, 9000], u[:, 9000] = sign * lo, 0.25
+    ref = _oracle(x, T, u)
+    assert (ref[0] == 10).all()
+    for got in _run(torch.from_numpy(x).to(cuda), torch.full((B,), T, device=cuda),
+                    uniforms=torch.from_numpy(u).to(cuda)):
+        _same(got, ref)
+
+
 def test_plain_oracle(cuda):
     """Full-size rows against the sequential oracle (given uniforms), the whole batch twice (the
     arrival counters are left ready)."""

@@ -10,8 +10,8 @@
 // largest seen (a handful), delta a bound on the rounding of both forms, and the part that
 // arrives last computes the exact keys of those alone, with the row maximum known.  A row takes
 // the multi-pass sampler's two passes of exact keys (exact_row) only when the short lists cannot
-// decide it (no finite maximum, uniforms outside [0, 1), more near-equal keys than a list holds, a
-// best key near underflow).
+// decide it (no finite maximum, or one whose x c is at the edge of fp32's range, uniforms outside
+// [0, 1), more near-equal keys than a list holds, a best key near underflow).
 //
 // Bound: VALU, by the generated uniforms (Philox-4x32-10: 20 quarter-rate 32 x 32 multiplies per
 // four tokens).  E >= 1 - u >= 2^-24 gives each block of four tokens the bound max x c + 24, so
@@ -424,7 +424,10 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     }
     const float m = maxk ? val_of(maxk) / Tt : __builtin_nanf("");
     const bool fin = m > -__builtin_inff() && m < __builtin_inff();
-    if (!fin || over || ntot == 0u) {  // (uniform)
+    // x c of the largest logits at the edge of fp32's range: it can be infinite for one of two
+    // neighbours that y holds equal, and g orders nothing there
+    const bool past = !(__builtin_fabsf(val_of(maxk) * c) < 0x1p127f);
+    if (!fin || past || over || ntot == 0u) {  // (uniform)
         exact_row<T>(a, sm, r, row, Tt, maxk);
         return;
     }
@@ -441,8 +444,8 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     plain_merge(sm, rr);
     // A key below 2^-91 decides nothing: exp_det is 0 below -80, so an element whose exact key is 0
     // can have g only 80 log2(e) - 24 = 91.4 below the row maximum's x c (E >= 2^-24), and hide a
-    // better live one of its part (the largest logits drew u = 0, or a part's x c overflowed and
-    // its list is empty).  From 2^-91 on no exponential in reach is 0 and g orders the keys.
+    // better live one of its part (where the largest logits drew u = 0).  From 2^-91 on no
+    // exponential in reach is 0 and g orders the keys.
     const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-91f;
     if (tid == 0) sm.last = won ? 1u : 0u;
     if (tid == 0 && won)

@@ -170,6 +170,31 @@ def test_scaled_logits_at_the_edge_of_their_range(cuda, sign):
         _same(got, ref)
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("V", [3, 4099, 16385])
+def test_infinite_temperature(cuda, dtype, V):
+    """T = +inf makes every finite logit 0 and every infinite one NaN: not counted among the
+    survivors, never drawn; rows of infinities alone return their first token."""
+    import torch
+
+    B = 6
+    xd, g = _logits(cuda, B, V, dtype, seed=5)
+    xd[1, 1:] = -float("inf")
+    xd[2, V - 2] = float("inf")
+    xd[3] = float("inf")
+    xd[4, ::2] = float("nan")
+    xd[4, 1] = -float("inf")
+    xd[5] = -float("inf")
+    u = torch.randint(1, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24
+    with np.errstate(invalid="ignore"):
+        ref = _oracle(xd.float().cpu().numpy(), np.inf, u.cpu().numpy())
+    T = torch.full((B,), float("inf"), device=cuda)
+    _same(*_run(xd, T, both=False, uniforms=u), ref)
+    xd[2, V - 2] = 0.0  # (a +inf logit among finite ones is the plain kernel's and the oracle's case only)
+    _same(*_run(xd, T, uniforms=u))
+    _same(*_run(xd, T, rng_key=99))
+
+
 def test_plain_oracle(cuda):
     """Full-size rows against the sequential oracle (given uniforms), the whole batch twice (the
     arrival counters are left ready)."""

@@ -11,7 +11,7 @@
 // arrives last computes the exact keys of those alone, with the row maximum known.  A row takes
 // the multi-pass sampler's two passes of exact keys (exact_row) only when the short lists cannot
 // decide it (no finite maximum, or one whose x c is at the edge of fp32's range, uniforms outside
-// [0, 1), more near-equal keys than a list holds, a best key near underflow).
+// [0, 1), more near-equal keys than a list holds, a best key near underflow, an infinite temperature).
 //
 // Bound: VALU, by the generated uniforms (Philox-4x32-10: 20 quarter-rate 32 x 32 multiplies per
 // four tokens).  E >= 1 - u >= 2^-24 gives each block of four tokens the bound max x c + 24, so
@@ -143,8 +143,15 @@ template <typename T>
 __device__ __forceinline__ void exact_row(const PlainArgs& a, PlainSmem& sm, int r, const T* row, float Tt,
                                           uint32_t maxk) {
     const int tid = threadIdx.x;
-    const float m = maxk ? val_of(maxk) / Tt : __builtin_nanf("");
+    float m = maxk ? val_of(maxk) / Tt : __builtin_nanf("");
     RowRace rs;
+    if (Tt == __builtin_inff()) {
+        // y is 0 for a finite logit and NaN for an infinite one, the largest among them
+        int any = 0;
+        for (int i = tid; i < a.V; i += kPlThreads)
+            any |= __builtin_fabsf(Elem<T>::load1(row + i)) < __builtin_inff() ? 1 : 0;
+        m = __syncthreads_or(any) ? 0.0f : __builtin_nanf("");
+    }
     if (!(m > -__builtin_inff() && m < __builtin_inff())) {
         const uint32_t km = key_of(m);
         for (int i = tid; i < a.V; i += kPlThreads)
@@ -427,7 +434,8 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     // x c of the largest logits at the edge of fp32's range: it can be infinite for one of two
     // neighbours that y holds equal, and g orders nothing there
     const bool past = !(__builtin_fabsf(val_of(maxk) * c) < 0x1p127f);
-    if (!fin || past || over || ntot == 0u) {  // (uniform)
+    // (an infinite temperature turns infinite logits into NaN, which the counts above miss)
+    if (!fin || past || over || ntot == 0u || Tt == __builtin_inff()) {  // (uniform)
         exact_row<T>(a, sm, r, row, Tt, maxk);
         return;
     }

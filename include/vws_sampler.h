@@ -188,7 +188,7 @@ int32_t vws_abi_version(void);
 const char* vws_last_error(void);
 
 /* Bytes of workspace vws_sample needs for this shape and history width
- * (prompt_width + output_width + adjust_width): a fixed region (about 670 KiB, first) through
+ * (prompt_width + output_width + adjust_width): a fixed region (about 740 KiB, first) through
  * which the workgroups of one launch share the extra passes over a row's logits that some
  * top-p rows need, and through which a batch larger than the device's resident workgroups
  * gets its rows handed out; then the history hash of rows served by the multi-pass path,

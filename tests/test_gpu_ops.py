@@ -100,3 +100,39 @@ def test_penalties_then_topk_then_sample_shared_workspace(cuda):
             assert np.array_equal(vals.cpu().numpy(), rv), f"round {rnd} k {k}: values"
         w = W.config(3, scale=0.1)
         assert_same(gpu_run(w, cuda), oracle_run(w), f"round {rnd}: sample after topk")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_topk_batches_of_different_size_share_a_workspace(cuda, dtype):
+    """Regression: where a batch's arrival counters ended and its part records began depended on
+    the batch, so a small batch left its records in a larger one's counters (rows from 128 on
+    elected no last part and returned uninitialised memory)."""
+    import torch
+
+    from vllm_webgpu_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(5)
+    for B, V, k in ((300, 20011, 40), (16, 20011, 256), (300, 20011, 40), (1, 150001, 3), (700, 9001, 7),
+                    (16, 70001, 100), (300, 20011, 256)):
+        x = torch.randn((B, V), generator=g, device=cuda)
+        if B == 16:
+            x[5:9] = 1.0  # (rows whose lists overflow: handed to the second kernel)
+        x = x.to(torch.float32 if dtype == "f32" else torch.bfloat16)
+        vals, ids = ops.topk(x, k)
+        want, order = torch.sort(x.float(), dim=1, descending=True, stable=True)
+        assert torch.equal(vals, want[:, :k]) and torch.equal(ids.long(), order[:, :k]), (B, V, k)
+
+
+@pytest.mark.parametrize("B,V", [(8192, 300), (8193, 300), (16390, 8200), (8200, 33000)])
+def test_topk_more_rows_than_a_launch(cuda, B, V):
+    """Batches at and past the 8192 rows one launch takes, in one part and in several."""
+    import torch
+
+    from vllm_webgpu_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(B)
+    x = torch.randn((B, V + 3), generator=g, device=cuda)[:, :V]
+    vals, ids = ops.topk(x, 5)
+    assert torch.equal(vals, torch.topk(x, 5, dim=1).values)
+    assert torch.equal(torch.gather(x, 1, ids.long()), vals)
+    assert (torch.sort(ids, dim=1).values.diff(dim=1) > 0).all()

@@ -38,10 +38,11 @@ using namespace vws;
 // Static device scratch of vws_sample_noalloc (one copy per GPU, held until the process ends).
 // Host code never uses this name as an address: the per-device address comes from
 // hipGetSymbolAddress (scratch_address below) and only that pointer is handed to kernels.
-// The plain rows' records come on top of the documented size, so that they leave the accepted
-// batches as they are.
-constexpr size_t kPlainBytes = sizeof(CoopState::plain_ctr) + sizeof(CoopState::plain_rec);
-constexpr size_t kScratchBytes = VWS_NOALLOC_SCRATCH_BYTES + kPlainBytes;
+// The plain rows' records and the top-k's counters come on top of the documented size, so that
+// they leave the accepted batches as they are.
+constexpr size_t kExtraBytes = sizeof(CoopState::plain_ctr) + sizeof(CoopState::plain_rec) +
+                               sizeof(CoopState::topk_ctr) + sizeof(CoopState::topk_state);
+constexpr size_t kScratchBytes = VWS_NOALLOC_SCRATCH_BYTES + kExtraBytes;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
@@ -302,8 +303,9 @@ KArgs make_kargs(int B, int V, const void* logits, int64_t stride, void* ws, int
     const WsLayout w = ws_layout(B, V, hw, parts);
     char* base = static_cast<char*>(ws);
     if (parts) {
-        k.row_counter = reinterpret_cast<uint32_t*>(base + w.counter);
-        k.row_state = reinterpret_cast<uint32_t*>(base + w.state);
+        CoopState* st = reinterpret_cast<CoopState*>(base + w.coop);
+        k.row_counter = st->topk_ctr;
+        k.row_state = st->topk_state;
         k.part_meta = reinterpret_cast<uint32_t*>(base + w.meta);
         k.part_list = reinterpret_cast<uint2*>(base + w.list);
     }
@@ -622,29 +624,34 @@ int vws_topk(const void* logits, int32_t dtype, int32_t batch, int32_t vocab, in
     const size_t need = vws_topk_workspace_size(batch, vocab, k);
     if (!workspace || workspace_bytes < need)
         return fail(VWS_ERR_WORKSPACE_TOO_SMALL, "workspace has %zu bytes, need %zu", workspace_bytes, need);
-    KArgs ka = make_kargs(batch, vocab, logits, row_stride, workspace, 0, true);
-    ka.topk_k = k;
-    ka.topk_vals = out_vals;
-    ka.topk_ids = out_ids;
-    choose_parts(batch, vocab, k, &ka.S, &ka.part_len);
+    const size_t row_bytes = (size_t)row_stride * (dtype == VWS_DTYPE_F32 ? 4 : 2);
     hipStream_t s = (hipStream_t)stream;
-    const int bp = (batch + 7) / 8 * 8;
     const int K = VWS_KERNEL_TOPK;
-    if (dtype == VWS_DTYPE_F32)
-        launch(K, fast_kernel<float>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
-    else if (dtype == VWS_DTYPE_BF16)
-        launch(K, fast_kernel<uint16_t>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
-    else
-        launch(K, fast_kernel<_Float16>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
-    if ((st = check_launch("vws_topk"))) return st;
-    // rows whose single-pass candidate lists overflowed (ties) are finished exactly here
-    if (dtype == VWS_DTYPE_F32)
-        launch(K, general_kernel<float>, dim3(batch), dim3(kGenThreads), s, ka);
-    else if (dtype == VWS_DTYPE_BF16)
-        launch(K, general_kernel<uint16_t>, dim3(batch), dim3(kGenThreads), s, ka);
-    else
-        launch(K, general_kernel<_Float16>, dim3(batch), dim3(kGenThreads), s, ka);
-    if ((st = check_launch("vws_topk (general kernel)"))) return st;
+    for (int r0 = 0; r0 < batch; r0 += kTopkRows) {
+        const int rows = batch - r0 < kTopkRows ? batch - r0 : kTopkRows;
+        KArgs ka = make_kargs(rows, vocab, static_cast<const char*>(logits) + (size_t)r0 * row_bytes, row_stride,
+                              workspace, 0, true);
+        ka.topk_k = k;
+        ka.topk_vals = out_vals + (size_t)r0 * k;
+        ka.topk_ids = out_ids + (size_t)r0 * k;
+        choose_parts(rows, vocab, k, &ka.S, &ka.part_len);
+        const int bp = (rows + 7) / 8 * 8;
+        if (dtype == VWS_DTYPE_F32)
+            launch(K, fast_kernel<float>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
+        else if (dtype == VWS_DTYPE_BF16)
+            launch(K, fast_kernel<uint16_t>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
+        else
+            launch(K, fast_kernel<_Float16>, dim3(bp * ka.S), dim3(kFastThreads), s, ka);
+        if ((st = check_launch("vws_topk"))) return st;
+        // rows whose single-pass candidate lists overflowed (ties) are finished exactly here
+        if (dtype == VWS_DTYPE_F32)
+            launch(K, general_kernel<float>, dim3(rows), dim3(kGenThreads), s, ka);
+        else if (dtype == VWS_DTYPE_BF16)
+            launch(K, general_kernel<uint16_t>, dim3(rows), dim3(kGenThreads), s, ka);
+        else
+            launch(K, general_kernel<_Float16>, dim3(rows), dim3(kGenThreads), s, ka);
+        if ((st = check_launch("vws_topk (general kernel)"))) return st;
+    }
     return ok();
 }
 

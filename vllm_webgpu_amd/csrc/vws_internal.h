@@ -18,6 +18,7 @@ constexpr int kPartCap = 512;                     // list entries a part may pub
 constexpr int kMergeCap = kFastWaves * kCapW;     // entries the last part can merge
 constexpr int kPartMax = 32768;                   // elements per part
 constexpr int kMaxParts = 16;                    // parts per row: VWS_MAX_VOCAB / kPartMax
+constexpr int kTopkRows = 8192;                  // rows per launch (their counters' places in CoopState)
 
 // Plain rows (vws_plain.hip): threads per part, most parts of a row, and the records of a launch
 // (parts of all its rows) the workspace holds.
@@ -105,6 +106,11 @@ struct CoopState {
     // plain rows split over several workgroups: parts arrived per row (left at zero) and records
     uint32_t plain_ctr[kPlRecs];
     uint64_t plain_rec[(size_t)kPlRecs * 8];
+    // split top-k: parts arrived per row and rows left to general_kernel (both left at zero).
+    // They lie here, and not where a batch's part lists end, because what one launch leaves in
+    // its lists must never be another's counter, whatever their batches.
+    uint32_t topk_ctr[kTopkRows];
+    uint32_t topk_state[kTopkRows];
 };
 
 struct KArgs {
@@ -152,8 +158,8 @@ struct KArgs {
     float* lp_vals;
     int32_t* lp_ranks;
     // workspace views
-    uint32_t* row_counter;  // [B]
-    uint32_t* row_state;    // [B]
+    uint32_t* row_counter;  // [B] (CoopState::topk_ctr)
+    uint32_t* row_state;    // [B] (CoopState::topk_state)
     uint32_t* part_meta;    // [B * kMaxParts * 4]: count, kth key, status, 0
     uint2* part_list;       // [B * kMaxParts * kPartCap]: (key, index)
     uint32_t* hist_hash;    // [B * hs_row * 4]: token+1, count | flags, penalised bits, bias
@@ -177,7 +183,7 @@ struct KArgs {
 
 // Workspace layout (bytes, 256-aligned sections).
 struct WsLayout {
-    size_t counter, state, meta, list, coop, hash, total;
+    size_t meta, list, coop, hash, total;
     int hs_row;
 };
 
@@ -192,17 +198,16 @@ inline int hash_slots_for(int history_width) {
 
 // Workspace sections.  Every layout starts with the cooperative-pass region at offset 0, so that
 // one workspace can serve every operation in turn (the region keeps its state between sampling
-// calls; the other operations leave it alone).  Then: sampling and the penalty op, the history
-// hash of the multi-pass path (B x hs_row x 4 words); the split top-k op (parts = true), its
-// per-row counters, row states and part lists.
+// calls; the top-k op keeps its counters there, the others leave it alone).  Then: sampling and
+// the penalty op, the history hash of the multi-pass path (B x hs_row x 4 words); the split top-k
+// op (parts = true), its part records and lists.  What follows the region may hold anything.
 inline WsLayout ws_layout(int B, int V, int history_width, bool parts) {
     (void)V;
     WsLayout w{};
     size_t off = 0;
     w.coop = off;    off = align256(off + sizeof(CoopState));
     if (parts) {
-        w.counter = off; off = align256(off + sizeof(uint32_t) * (size_t)B);
-        w.state = off;   off = align256(off + sizeof(uint32_t) * (size_t)B);
+        if (B > kTopkRows) B = kTopkRows;  // (launched kTopkRows rows at a time)
         w.meta = off;    off = align256(off + sizeof(uint32_t) * 4 * (size_t)B * kMaxParts);
         w.list = off;    off = align256(off + sizeof(uint2) * (size_t)B * kMaxParts * kPartCap);
     }

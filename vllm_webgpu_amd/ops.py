@@ -20,9 +20,9 @@ import torch
 from . import _lib
 
 _ws_lock = threading.Lock()
-_ws_cache: dict[int, torch.Tensor] = {}               # by device
-_ws_side: dict[tuple[int, int], torch.Tensor] = {}    # by device and stream, other than the default stream
-_WS_SIDE_MAX = 32
+_ws_cache: dict[int, torch.Tensor] = {}               # the default stream's, by device
+_ws_side: dict[tuple[int, int], torch.Tensor] = {}    # other streams', by device and stream
+_WS_SIDE_MAX = 64                                     # of those; the oldest is dropped
 
 
 def _stream_ptr() -> int:
@@ -74,10 +74,35 @@ def _history(ids, lens, B: int, device, name: str):
     return ids, ids.stride(0), ids.shape[1], lens
 
 
-def _new_workspace(nbytes: int, idx: int) -> torch.Tensor:
-    ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=f"cuda:{idx}")
-    _lib.check(_lib.lib().vws_workspace_init(ws.data_ptr(), ws.numel(), _stream_ptr()))
+def _capturing(stream: int) -> bool:
+    # (the default stream is never captured)
+    return stream != 0 and torch.cuda.is_current_stream_capturing()
+
+
+def _new_workspace(nbytes: int, clear: int, idx: int, stream: int) -> torch.Tensor:
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=f"cuda:{idx}")
+    _lib.check(_lib.lib().vws_workspace_init(ws.data_ptr(), clear, stream))
     return ws
+
+
+def _workspace(nbytes: int, idx: int, stream: int, capturing: bool) -> torch.Tensor:
+    if capturing:
+        # a buffer for this call alone, cleared by the graph at each replay (the fixed region,
+        # which is what must be clean)
+        fixed = _lib.lib().vws_sample_workspace_size(1, 1, 0)
+        return _new_workspace(nbytes, min(nbytes, fixed), idx, stream)
+    cache, key = (_ws_side, (idx, stream)) if stream else (_ws_cache, idx)
+    ws = cache.get(key)
+    if ws is not None and ws.numel() >= nbytes:
+        return ws
+    with _ws_lock:
+        size = max(nbytes, 1 << 20)
+        ws = _new_workspace(size, size, idx, stream)
+        cache.pop(key, None)
+        if stream and len(cache) >= _WS_SIDE_MAX:
+            del cache[next(iter(cache))]
+        cache[key] = ws
+        return ws
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
@@ -85,30 +110,17 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     that stream.
 
     The kernels leave the buffer clean for the next call but do not guard concurrent use (the
-    parts of a split row count their arrivals there), so calls that may overlap need buffers of
-    their own: each stream has one, up to ``_WS_SIDE_MAX`` streams besides the default one; calls
-    on further streams, and calls under graph capture on a stream without one, share the device's
-    and must run in stream order with its other users.
+    parts of a split row count their arrivals there), so each stream has a buffer of its own.
+    A buffer that is dropped (outgrown, or the oldest of more than ``_WS_SIDE_MAX``) goes back to
+    torch's allocator, which hands it out again in the order of the stream that used it.
+
+    Under graph capture each call gets a buffer that nothing else uses and that the graph clears:
+    a replay may overlap any stream's eager calls.  Its memory is the capture's (torch gives the
+    allocations of a capture to the graph's own pool), not the cache's.
     """
     idx = device.index if device.index is not None else torch.cuda.current_device()
     stream = torch._C._cuda_getCurrentRawStream(idx)
-    with _ws_lock:
-        if stream:
-            ws = _ws_side.get((idx, stream))
-            if ws is not None and ws.numel() >= nbytes:
-                return ws
-            if not torch.cuda.is_current_stream_capturing():
-                if ws is not None or len(_ws_side) < _WS_SIDE_MAX:
-                    ws = _ws_side[idx, stream] = _new_workspace(nbytes, idx)
-                    return ws
-        ws = _ws_cache.get(idx)
-        if ws is None or ws.numel() < nbytes:
-            if stream:  # one that a warm-up on another stream has made, rather than a new one
-                for (i, _), w in _ws_side.items():
-                    if i == idx and w.numel() >= nbytes:
-                        return w
-            ws = _ws_cache[idx] = _new_workspace(nbytes, idx)
-        return ws
+    return _workspace(nbytes, idx, stream, _capturing(stream))
 
 
 @dataclass
@@ -125,24 +137,36 @@ class PreparedSample:
     """One ``vws_sample`` call with its arguments validated and packed once (``prepare_sample``):
     ``launch()`` issues it again on the current stream with one C call, reading the same input
     tensors (their current contents) and writing the same ``result`` tensors.  The object keeps
-    every tensor it points at alive, the workspace of the stream it was prepared on among them:
-    launches on another stream must be in order with that stream's calls."""
+    every tensor it points at alive, the workspace of the stream it was prepared on among them;
+    a launch on another stream, or into a graph, uses that stream's or that graph's workspace."""
 
-    def __init__(self, args, result: SampleResult, keep: tuple):
+    def __init__(self, args, result: SampleResult, keep: tuple, stream: int | None = None,
+                 ws_bytes: int = 0, device_index: int = 0):
         self.args = args
         self.result = result
         self._keep = keep
+        self._stream = stream  # the stream whose workspace ``args`` holds (None: a graph's)
+        self._ws_bytes = ws_bytes
+        self._device_index = device_index
 
     def launch(self) -> SampleResult:
-        self.args.stream = _stream_ptr()
-        _lib.check(_lib.lib().vws_sample(ctypes.byref(self.args)))
+        stream = _stream_ptr()
+        args, ws = self.args, None
+        capturing = _capturing(stream)
+        if stream != self._stream or capturing:
+            args = _lib.SampleArgs.from_buffer_copy(args)
+            ws = _workspace(self._ws_bytes, self._device_index, stream, capturing)
+            args.workspace, args.workspace_bytes, args.stream = ws.data_ptr(), ws.numel(), stream
+        _lib.check(_lib.lib().vws_sample(ctypes.byref(args)))
         return self.result
 
 
 def sample(logits: torch.Tensor, *args, **kwargs) -> SampleResult:
     """Samples one token per row of ``logits`` [B, V] (float32, bfloat16 or float16, on the
     GPU; each widened exactly to fp32).  Arguments: those of ``prepare_sample``."""
-    return prepare_sample(logits, *args, **kwargs).launch()
+    call = prepare_sample(logits, *args, **kwargs)  # (its arguments hold the current stream)
+    _lib.check(_lib.lib().vws_sample(ctypes.byref(call.args)))
+    return call.result
 
 
 def prepare_sample(logits: torch.Tensor, temperature=None, top_k=None, top_p=None, min_p=None,
@@ -262,7 +286,9 @@ def prepare_sample(logits: torch.Tensor, temperature=None, top_k=None, top_p=Non
         ranks = torch.empty(B, dtype=torch.int32, device=dev)
     L_lib = _lib.lib()
     nbytes = L_lib.vws_sample_workspace_size(B, V, pwidth + owidth + awidth)
-    ws = workspace(nbytes, dev)
+    stream = _stream_ptr()
+    capturing = _capturing(stream)
+    ws = _workspace(nbytes, dev.index, stream, capturing)
     a = _lib.SampleArgs()
     a.struct_size = ctypes.sizeof(_lib.SampleArgs)
     a.batch, a.vocab, a.dtype = B, V, _dtype_code(logits)
@@ -290,10 +316,11 @@ def prepare_sample(logits: torch.Tensor, temperature=None, top_k=None, top_p=Non
     a.sampled, a.row_flags, a.num_kept = sampled.data_ptr(), flags.data_ptr(), nkept.data_ptr()
     a.num_logprobs = L
     a.logprob_ids, a.logprob_vals, a.logprob_ranks = _ptr(lp_ids), _ptr(lp_vals), _ptr(ranks)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    a.workspace, a.workspace_bytes, a.stream = ws.data_ptr(), ws.numel(), stream
     keep = (logits, T, K, P, MP, R, PR, FR, pid, plens, oid, olens, aid, aval, alens, TS, TR,
             token_state_bits, AM, U, SEED, OFF, ws)
-    return PreparedSample(a, SampleResult(sampled, flags, nkept, lp_ids, lp_vals, ranks), keep)
+    return PreparedSample(a, SampleResult(sampled, flags, nkept, lp_ids, lp_vals, ranks), keep,
+                          None if capturing else stream, nbytes, dev.index)
 
 
 def token_state_update(state: torch.Tensor, tokens: torch.Tensor, rows=None, prompt: bool = False,

@@ -197,9 +197,10 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     const int nblk = a.V >> 2;
     const int b0 = p * a.part_blocks, b1 = min(nblk, b0 + a.part_blocks);
     const bool dword = (reinterpret_cast<uintptr_t>(row) & 3u) == 0u;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, (uint32_t)nblk * 4u * (uint32_t)sizeof(T));
+    // (the resources end with the part: what is asked for past it is zeros and not fetched)
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, (uint32_t)b1 * 4u * (uint32_t)sizeof(T));
     const __amdgpu_buffer_rsrc_t us = make_rsrc(gen ? (const void*)row : (const void*)urow,
-                                                gen ? 0u : (uint32_t)nblk * 16u);
+                                                gen ? 0u : (uint32_t)b1 * 16u);
     if (tid == 0) { sm.ncand = 0u; sm.nsel = 0u; sm.bad = 0u; sm.thr = 0u; sm.maxk = 0u; sm.count = 0u; }
     __syncthreads();
 
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     };
     load(X, 0);
     for (int it = 0; it < nit; ++it) {
-        load(Y, it + 1);  // (past the row's blocks: zeros, nothing fetched)
+        load(Y, it + 1);  // (past the part's blocks: zeros, nothing fetched)
 #pragma unroll
         for (int q = 0; q < kPlBlocks; ++q) {
             const int b = b0 + (it * kPlBlocks + q) * kPlThreads + tid;

@@ -195,6 +195,41 @@ def test_infinite_temperature(cuda, dtype, V):
     _same(*_run(xd, T, rng_key=99))
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("V", [1, 3, 6, 1024, 8193, 40003, 262147])
+def test_exact_rows(cuda, dtype, V):
+    """Rows read again for their exact keys (a uniform outside [0, 1) or NaN, in the first, the last
+    and other tokens) and for the first token of their maximum (infinities at every place, NaN
+    before them, y = x / T that overflows), odd starts and remainders, one part and several."""
+    import torch
+
+    B = 16
+    xw, g = _logits(cuda, B, V + 1, dtype, seed=6)
+    x = xw[:, 1:] if V > 1 else xw[:, :1].contiguous()
+    u = torch.randint(1, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24
+    T = torch.exp(torch.linspace(-3.0, 3.0, B, device=cuda))
+    inf, nan, at = float("inf"), float("nan"), torch.randint(0, V, (B,), generator=g, device=cuda).tolist()
+    for r, v in ((0, 1.0), (1, nan), (2, -0.5), (3, 1.0), (4, 2.0), (5, inf)):
+        u[r, at[r]] = v
+    u[3, :] = 1.0
+    u[6, 0] = u[6, V - 1] = 1.0
+    u[7, V - 1] = nan
+    x[8, at[8]] = inf
+    x[9, at[9]:] = inf
+    x[10, V - 1] = x[10, V // 2] = inf
+    x[10, : V // 2] = nan
+    x[11] = -inf
+    x[12, : V // 2] = nan
+    x[12, V // 2 :] = -inf
+    x[13] = nan
+    if dtype != "f16":
+        T[14] = T[15] = 0.25
+        x[14, at[14]] = 0.9 * torch.finfo(x.dtype).max
+        x[15, max(0, V - 3) :] = 0.9 * torch.finfo(x.dtype).max
+    _same(*_run(x, T, uniforms=u))
+    _same(*_run(x[8:], T[8:], rng_key=5))
+
+
 def test_plain_oracle(cuda):
     """Full-size rows against the sequential oracle (given uniforms), the whole batch twice (the
     arrival counters are left ready)."""

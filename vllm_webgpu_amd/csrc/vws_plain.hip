@@ -8,10 +8,10 @@
 //     log2 key_i = x_i c - log2 E_i - const,  c = log2(e) / T,
 // so each part of a row keeps the elements whose g_i = x_i c - log2 E_i lies within delta of the
 // largest seen (a handful), delta a bound on the rounding of both forms, and the part that
-// arrives last computes the exact keys of those alone, with the row maximum known.  A row takes
-// the multi-pass sampler's two passes of exact keys (exact_row) only when the short lists cannot
-// decide it (no finite maximum, or one whose x c is at the edge of fp32's range, uniforms outside
-// [0, 1), more near-equal keys than a list holds, a best key near underflow, an infinite temperature).
+// arrives last computes the exact keys of those alone, with the row maximum known.  It reads the
+// row again (exact_row) only when the short lists cannot decide it: no finite maximum, or one
+// whose x c is at the edge of fp32's range, uniforms outside [0, 1), more near-equal keys than a
+// list holds, a best key near underflow, an infinite temperature.
 //
 // Bound: VALU, by the generated uniforms (Philox-4x32-10: 20 quarter-rate 32 x 32 multiplies per
 // four tokens).  E >= 1 - u >= 2^-24 gives each block of four tokens the bound max x c + 24, so
@@ -19,8 +19,8 @@
 // them fill its lanes; per token one hardware log2 of 1 - u (E >= 1 - u: an upper bound of g)
 // decides whether log_det and the second log2 are computed at all.  128 rows of 151936 bf16
 // logits: 257 us on the multi-pass path (one workgroup per row, three transcendental sequences
-// and a division per element) -> 33.5 us; 4 rows 244 -> 12.1 us; 256 rows of fp32 with given uniforms
-// (read whole: 311 MB) 227 -> 56 us.
+// and a division per element) -> 30.3 us; 4 rows 244 -> 11.6 us; 256 rows of fp32 with given uniforms
+// (read whole: 311 MB) 227 -> 55 us.
 #include "vws_plain.h"
 
 namespace vws {
@@ -41,6 +41,8 @@ struct PlainSmem {
     uint32_t count;
     uint64_t red[kPlWaves][3];
 };
+
+__shared__ PlainSmem g_plain_sh;
 
 // A part's record: words 0 (largest key << 32 | NaN elements), 1 (candidates, or
 // kPlOver) and 2-7 (candidates: token << 32 | logit bits).  Greedy rows: word 0 the best
@@ -137,50 +139,183 @@ __device__ __forceinline__ void plain_merge(PlainSmem& sm, RowRace& rs) {
     }
 }
 
-// A row the lists cannot decide, by one workgroup: the row maximum is maxk; every element's exact
-// key (or, without a finite maximum, the first index of the largest key of y).
+// A row the lists cannot decide, by one workgroup: the row maximum is maxk; the best exact key (or,
+// without a finite maximum, the first index of the largest key of y).  Only rows without a
+// finite maximum, with uniforms outside [0, 1) or with very many near-equal keys come here in
+// earnest.
+//
+// One workgroup reads the row again, so it is bound by the latency of its loads (EX blocks per lane,
+// twice, in flight) and, where the keys decide, by their arithmetic: once an exact key of at
+// least 2^-91 is known (see plain_kernel), an element whose bound of g (E >= 1 - u, and before the
+// uniforms are generated E >= 2^-24) is below that key's g and delta is not computed; one whose
+// uniform is outside [0, 1), which the bound does not hold for, always is.  Reading one element per
+// load and computing every key it took 128 rows of 151936 bf16 logits with a +inf 343 us (55 now)
+// and 128 of 128256 fp32 with a uniform of 1 each 587 us (152 now; the multi-pass path 85 and 158).
+//
+// A function of its own (which reads the kernel's arguments again), so that its registers and code
+// stay out of the kernel: 128 rows of 151936 bf16 logits none of which comes here 32.9 -> 30.3 us,
+// 256 x 151936 fp32 with given uniforms 55.1 -> 55.2.
 template <typename T>
-__device__ __forceinline__ void exact_row(const PlainArgs& a, PlainSmem& sm, int r, const T* row, float Tt,
-                                          uint32_t maxk) {
-    const int tid = threadIdx.x;
+__device__ __noinline__ void exact_row(uint64_t kernarg, int r, uint32_t maxk) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using ArgsConst = const PlainArgs __attribute__((address_space(4)));
+    const uint64_t ka = ((uint64_t)tp_first((uint32_t)(kernarg >> 32)) << 32) | tp_first((uint32_t)kernarg);
+    const PlainArgs a = *(ArgsConst*)ka;
+    r = (int)tp_first((uint32_t)r);
+    maxk = tp_first(maxk);
+    PlainSmem& sm = g_plain_sh;
+    const T* row = reinterpret_cast<const T*>(a.logits) + (size_t)r * a.lstride;
+    const float Tt = a.temperature[r];  // (no greedy row comes here)
+    const float c = kPlLog2e / Tt;
+    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int EX = sizeof(T) == 4 ? 4 : 8;  // (8 of fp32 would leave the kernel two workgroups a CU)
+    const int nblk = a.V >> 2;
+    const int nit = (nblk + kPlThreads * EX - 1) / (kPlThreads * EX);
+    const bool dword = (reinterpret_cast<uintptr_t>(row) & 3u) == 0u;
+    const bool gen = a.u == nullptr;
+    const float inf = __builtin_inff();
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, (uint32_t)nblk * 4u * (uint32_t)sizeof(T));
+    const __amdgpu_buffer_rsrc_t us = make_rsrc(gen ? (const void*)row : (const void*)(a.u + (size_t)r * a.ustride),
+                                                gen ? 0u : (uint32_t)nblk * 16u);
+    if (tid == 0) sm.thr = 0u;
+    __syncthreads();
+    // f(x, t, ok) for every four tokens t .. t + 3, ascending in a lane: the row's blocks (ok: of
+    // the row), then the V % 4 tokens past them, the others NaN.  A wave goes on while f is true.
+    auto blocks = [&](auto f) __attribute__((always_inline)) {
+        float4 X[EX], Y[EX];
+        auto load = [&](float4 (&d)[EX], int it) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < EX; ++q)
+                d[q] = Block4<T>::load(rs, (uint32_t)((it * EX + q) * kPlThreads + tid), dword);
+        };
+        load(X, 0);
+        for (int it = 0; it < nit; ++it) {
+            load(Y, it + 1);
+#pragma unroll
+            for (int q = 0; q < EX; ++q) {
+                const int b = (it * EX + q) * kPlThreads + tid;
+                const float x[4] = {X[q].x, X[q].y, X[q].z, X[q].w};
+                if (!f(x, 4 * b, b < nblk)) return;
+            }
+#pragma unroll
+            for (int q = 0; q < EX; ++q) X[q] = Y[q];
+        }
+        if (tid < kWave && (a.V & 3)) {
+            const int t0 = nblk << 2;
+            float x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                x[j] = lane == 0 && t0 + j < a.V ? Elem<T>::load1(row + t0 + j) : __builtin_nanf("");
+            f(x, t0, lane == 0);
+        }
+    };
     float m = maxk ? val_of(maxk) / Tt : __builtin_nanf("");
-    RowRace rs;
-    if (Tt == __builtin_inff()) {
+    RowRace rr;
+    if (Tt == inf) {
         // y is 0 for a finite logit and NaN for an infinite one, the largest among them
         int any = 0;
-        for (int i = tid; i < a.V; i += kPlThreads)
-            any |= __builtin_fabsf(Elem<T>::load1(row + i)) < __builtin_inff() ? 1 : 0;
+        blocks([&](const float (&x)[4], int, bool ok) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) any |= ok && __builtin_fabsf(x[j]) < inf ? 1 : 0;
+            return wave_ballot(any != 0) == 0ull;
+        });
         m = __syncthreads_or(any) ? 0.0f : __builtin_nanf("");
     }
-    if (!(m > -__builtin_inff() && m < __builtin_inff())) {
-        const uint32_t km = key_of(m);
-        for (int i = tid; i < a.V; i += kPlThreads)
-            if (key_of(Elem<T>::load1(row + i) / Tt) == km) {
-                const uint64_t pk = 0x7FFFFFFFull - (uint32_t)i;  // (the lowest index has the largest)
-                rs.best = rs.best > pk ? rs.best : pk;
-            }
-        plain_merge(sm, rs);
-        if (tid == 0) plain_write(a, r, rs.best ? (int32_t)(0x7FFFFFFFu - (uint32_t)rs.best) : 0, VWS_FLAG_DEGENERATE, 1);
+    if (!(m > -inf && m < inf)) {
+        // the first token whose y is m: every y is NaN then (token 0), or every other one is
+        // -inf, or (y has overflowed) x c has nearly too
+        if (m == m)
+            blocks([&](const float (&x)[4], int t, bool ok) __attribute__((always_inline)) {
+                bool in[4], any = false;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    in[j] = ok && rr.best == 0ull && (m < 0.0f ? x[j] == x[j] : x[j] * c >= 0x1p127f);
+                    any = any || in[j];
+                }
+                if (wave_ballot(any) != 0ull) {
+#pragma unroll
+                    for (int j = 3; j >= 0; --j)  // (the lowest index has the largest, and is the lane's first)
+                        rr.best = in[j] && x[j] / Tt == m ? 0x7FFFFFFFull - (uint32_t)(t + j) : rr.best;
+                    if (rr.best) atomicMax(&sm.thr, (uint32_t)rr.best);
+                }
+                // (what follows in this wave lies past its first lane's tokens)
+                const uint32_t first = __hip_atomic_load(&sm.thr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                return tp_first(first) <= 0x7FFFFFFFu - tp_first((uint32_t)t);
+            });
+        plain_merge(sm, rr);
+        if (tid == 0) plain_write(a, r, rr.best ? (int32_t)(0x7FFFFFFFu - (uint32_t)rr.best) : 0, VWS_FLAG_DEGENERATE, 1);
         return;
     }
-    for (int i = tid; i < a.V; i += kPlThreads) {
-        const float y = Elem<T>::load1(row + i) / Tt;
-        const uint32_t ky = key_of(y);
-        if (!ky) continue;
-        const uint64_t lk = ((uint64_t)ky << 32) | (uint32_t)i;
-        rs.nkept++;
-        rs.last = rs.last > lk ? rs.last : lk;
-        rs.add_key(exp_det(y - m) / (0.0f - log_det(plain_uniform(a, r, i))), i);
-    }
-    plain_merge(sm, rs);
+    // whether g orders this row's keys (see plain_kernel)
+    const bool ordered = Tt < inf && __builtin_fabsf(val_of(maxk) * c) < 0x1p127f;
+    const uint64_t seed = gen ? (a.rng_seed ? a.rng_seed[r] : a.rng_key) : 0ull;
+    const uint64_t off = a.rng_seed ? (a.rng_offset ? a.rng_offset[r] : 0ull) : (uint64_t)(uint32_t)r;
+    float thr = -inf, lim = -inf;  // (wave-uniform)
+    blocks([&](const float (&x)[4], int t, bool ok) __attribute__((always_inline)) {
+        const float bm = __builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3]));
+        bool in[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            in[j] = ok && x[j] == x[j] && (Tt < inf || __builtin_fabsf(x[j]) < inf);  // (y is not NaN)
+            rr.nkept += in[j] ? 1u : 0u;
+        }
+        if (gen && wave_ballot(ok && !(__builtin_fmaf(bm, c, 24.0f) < lim)) == 0ull) return true;
+        float u[4];
+        if (gen) {
+            uint32_t k[4] = {(uint32_t)t >> 2, (uint32_t)off, (uint32_t)(off >> 32), 0u};
+            philox4x32_10(k, (uint32_t)seed, (uint32_t)(seed >> 32));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] = philox_word_uniform(k[j]);
+        } else if (t + 4 <= a.V) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b128(us, 4u * (uint32_t)t, 0u, 2);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] = u2f((uint32_t)w[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] = in[j] ? plain_uniform(a, r, t + j) : 0.5f;
+        }
+        bool need[4], any = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float z = __builtin_fmaf(x[j], c, -__builtin_amdgcn_logf(1.0f - u[j]));
+            need[j] = in[j] && !(u[j] >= 0.0f && u[j] < 1.0f && z < lim);
+            any = any || need[j];
+        }
+        if (wave_ballot(any) == 0ull) return true;
+        float top = -inf;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!need[j]) continue;
+            const float y = x[j] / Tt;
+            const uint64_t lk = ((uint64_t)key_of(y) << 32) | (uint32_t)(t + j);
+            rr.last = rr.last > lk ? rr.last : lk;
+            const float E = 0.0f - log_det(u[j]);
+            const float key = exp_det(y - m) / E;
+            rr.add_key(key, t + j);
+            if (u[j] < 1.0f && key >= 0x1p-91f) top = __builtin_fmaxf(top, __builtin_fmaf(x[j], c, -__builtin_amdgcn_logf(E)));
+        }
+        if (!ordered) return true;
+        const uint32_t st = tp_first(__hip_atomic_load(&sm.thr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        if (st) thr = __builtin_fmaxf(thr, val_of(st));
+        if (wave_ballot(top > thr)) {
+            thr = wave_max_f32(__builtin_fmaxf(top, thr));
+            if (lane == 0) atomicMax(&sm.thr, key_of(thr));
+        }
+        lim = thr - plain_delta(thr);
+        return true;
+    });
+    plain_merge(sm, rr);
     if (tid == 0)
-        plain_write(a, r, rs.best ? (int32_t)(0x7FFFFFFF - (uint32_t)rs.best) : (int32_t)(uint32_t)rs.last,
-                    plain_near_tie(rs), (int32_t)rs.nkept);
+        plain_write(a, r, rr.best ? (int32_t)(0x7FFFFFFF - (uint32_t)rr.best) : (int32_t)(uint32_t)rr.last,
+                    plain_near_tie(rr), (int32_t)rr.nkept);
+#else
+    (void)kernarg; (void)r; (void)maxk;
+#endif
 }
 
 template <typename T>
 __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
-    __shared__ PlainSmem sm;
+    PlainSmem& sm = g_plain_sh;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int S = a.S;
@@ -436,31 +571,33 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     // neighbours that y holds equal, and g orders nothing there
     const bool past = !(__builtin_fabsf(val_of(maxk) * c) < 0x1p127f);
     // (an infinite temperature turns infinite logits into NaN, which the counts above miss)
-    if (!fin || past || over || ntot == 0u || Tt == __builtin_inff()) {  // (uniform)
-        exact_row<T>(a, sm, r, row, Tt, maxk);
-        return;
+    bool exact = !fin || past || over || ntot == 0u || Tt == __builtin_inff();  // (uniform)
+    if (!exact) {
+        // exact keys of the listed candidates (6 slots a part)
+        RowRace rr;
+        for (int i = tid; i < S * 6; i += kPlThreads) {
+            const int q = i / 6, j = i - q * 6;
+            if (j >= (int)(uint32_t)sm.recs[q][1]) continue;
+            const uint64_t e = sm.recs[q][2 + j];
+            const int t = (int)(uint32_t)(e >> 32);
+            const float y = u2f((uint32_t)e) / Tt;
+            rr.add_key(exp_det(y - m) / (0.0f - log_det(plain_uniform(a, r, t))), t);
+        }
+        plain_merge(sm, rr);
+        // A key below 2^-91 decides nothing: exp_det is 0 below -80, so an element whose exact key is
+        // 0 can have g only 80 log2(e) - 24 = 91.4 below the row maximum's x c (E >= 2^-24), and hide
+        // a better live one of its part (where the largest logits drew u = 0).  From 2^-91 on no
+        // exponential in reach is 0 and g orders the keys.
+        const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-91f;
+        if (tid == 0) sm.last = won ? 1u : 0u;
+        if (tid == 0 && won)
+            plain_write(a, r, (int32_t)(0x7FFFFFFF - (uint32_t)rr.best), plain_near_tie(rr), (int32_t)count);
+        __syncthreads();
+        exact = !sm.last;
     }
-    // exact keys of the listed candidates (6 slots a part)
-    RowRace rr;
-    for (int i = tid; i < S * 6; i += kPlThreads) {
-        const int q = i / 6, j = i - q * 6;
-        if (j >= (int)(uint32_t)sm.recs[q][1]) continue;
-        const uint64_t e = sm.recs[q][2 + j];
-        const int t = (int)(uint32_t)(e >> 32);
-        const float y = u2f((uint32_t)e) / Tt;
-        rr.add_key(exp_det(y - m) / (0.0f - log_det(plain_uniform(a, r, t))), t);
-    }
-    plain_merge(sm, rr);
-    // A key below 2^-91 decides nothing: exp_det is 0 below -80, so an element whose exact key is 0
-    // can have g only 80 log2(e) - 24 = 91.4 below the row maximum's x c (E >= 2^-24), and hide a
-    // better live one of its part (where the largest logits drew u = 0).  From 2^-91 on no
-    // exponential in reach is 0 and g orders the keys.
-    const bool won = u2f((uint32_t)(rr.best >> 32)) >= 0x1p-91f;
-    if (tid == 0) sm.last = won ? 1u : 0u;
-    if (tid == 0 && won)
-        plain_write(a, r, (int32_t)(0x7FFFFFFF - (uint32_t)rr.best), plain_near_tie(rr), (int32_t)count);
-    __syncthreads();
-    if (!sm.last) exact_row<T>(a, sm, r, row, Tt, maxk);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (exact) exact_row<T>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr(), r, maxk);
+#endif
 }
 
 template __global__ void plain_kernel<float>(PlainArgs);

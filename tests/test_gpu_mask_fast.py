@@ -253,3 +253,36 @@ def test_logprob_launches_with_masks(cuda, case):
         lib.vws_set_single_pass(prev)
     assert_same(g2, ref, case + ", single pass off")
     assert ((g2["flags"][w.top_k > 0] & GENERAL) != 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_masked_topp_rows_that_start_unaligned_off_the_single_pass(cuda, dtype):
+    """Regression: with the single pass switched off, a masked top-p row that starts off a 16-byte
+    boundary went to the masked top-p stream, whose mask words line up with its vectors only on
+    one (bits of other tokens masked it)."""
+    import torch
+
+    from vllm_webgpu_amd import _lib, ops
+
+    B, V = 12, 32768
+    g = torch.Generator(device=cuda).manual_seed(5)
+    x = (torch.randn((B, V + 1), generator=g, device=cuda) * 2).to(
+        {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype])[:, 1:]
+    x[:, ::300] += 8.0
+    ok = torch.rand((B, V), generator=g, device=cuda) < 0.5
+    u = torch.randint(1, 1 << 24, (B, V), generator=g, device=cuda).float() * 2.0 ** -24
+    xm = x.float().masked_fill(~ok, -float("inf")).cpu().numpy()
+    one = np.ones(B, np.float32)
+    ref = O.sample(xm, O.make_params(B, 0.8 * one, np.zeros(B, np.int32), 0.9 * one, 0 * one, one, 0 * one, 0 * one),
+                   u.cpu().numpy())
+    T, P = torch.full((B,), 0.8, device=cuda), torch.full((B,), 0.9, device=cuda)
+    L = _lib.lib()
+    for on in (1, 0):
+        before = L.vws_set_single_pass(on)
+        try:
+            r = ops.sample(x, temperature=T, top_p=P, uniforms=u, allowed_mask=ops.pack_allowed(ok))
+            torch.cuda.synchronize()
+        finally:
+            L.vws_set_single_pass(before)
+        assert np.array_equal(r.sampled.cpu().numpy(), ref["token"])
+        assert np.array_equal(r.num_kept.cpu().numpy(), ref["n_kept"])

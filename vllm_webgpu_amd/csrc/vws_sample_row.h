@@ -2131,7 +2131,10 @@ __device__ __forceinline__ bool row_one(const KArgs& a, int r, const void* logit
                                         int V, uint64_t kernarg) {
     bool topp = false;
     if (a.nofast) {
-        topp = topp_eligible(a, row_params(a, r));
+        // (the masked stream takes rows that start 16-byte aligned, as row_fast's own test says)
+        Slice<T> sl;
+        if (XF == kXfMask) sl.init(static_cast<const T*>(logits) + (size_t)r * lstride, 0, V);
+        topp = topp_eligible(a, row_params(a, r)) && !(XF == kXfMask && sl.a != 0);
     } else if (row_fast<T, LP, XF == kXfMask>(a, g_row_sh.f, r, logits, lstride, V, &topp)) {
         if (!LP || row_logprobs_entry(r, kernarg)) return false;
     }

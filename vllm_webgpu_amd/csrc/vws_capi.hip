@@ -390,8 +390,10 @@ void softmax_launch(const T* logits, int B, int V, int64_t stride, const float* 
         launch(K, softmax_kernel<T>, dim3(B), dim3(1024), s, logits, stride, V, temperature, probs, row_max, log_sum);
         return;
     }
-    // parts of a multiple of 64 elements; the last one holds at least V / n - 63 (n - 1) of
+    // parts of a multiple of 64 elements; the last one holds at least V / n - 64 (n - 1) of
     // them, more than the 3 n words of the partial results its slice carries
+    static_assert(VWS_MAX_VOCAB <= kSmMaxParts * kSmPartMax && kSmMaxParts <= kWave,
+                  "softmax_write_kernel combines a row's parts one per lane");
     const int n = (V + kSmPartMax - 1) / kSmPartMax;
     const int len = ((V + n - 1) / n + 63) / 64 * 64;
     launch(K, softmax_part_kernel<T>, dim3(B * n), dim3(kSmThreads), s, logits, stride, V, len, n, temperature, probs);

@@ -116,10 +116,9 @@ def test_softmax(cuda):
 
 
 def test_softmax_long_rows(cuda):
-    """Rows longer than 32 values per thread (the two-read path: an online max and normaliser,
-    then the write), with -inf and NaN elements (exp_det is 0 for NaN: their probability is 0),
-    a row of one finite value, and a row in ascending order (every thread's running maximum
-    rises at each of its values)."""
+    """Rows of 19 parts (test_gpu_split_ops.py has the same kinds of row on the two-read path that rows
+    written over their logits take), with -inf and NaN elements (exp_det is 0 for NaN: their probability is 0),
+    a row of one finite value, and a row in ascending order."""
     import torch
 
     from vllm_webgpu_amd import ops

@@ -56,6 +56,43 @@ def test_softmax_over_its_logits(cuda, V):
     torch.testing.assert_close(x, want, rtol=1e-6, atol=1e-12)
 
 
+@pytest.mark.parametrize("V", [1, 2047, 2049, 8193, 32000, 32768, 32769, 150001])
+@pytest.mark.parametrize("inplace", [True, False])
+def test_softmax_one_workgroup_a_row(cuda, V, inplace):
+    """The forms of one workgroup per row, which rows above 2048 elements reach only where the
+    probabilities overlap the logits (held in registers up to 32768 less the row's edges, the
+    two-read path with its online maximum and normaliser above), against the oracle beside the
+    split form: -inf and NaN elements, a row of one finite value, ascending values (every
+    thread's maximum rises at each of its own), temperatures, the row maximum and log-sum."""
+    import torch
+
+    from oracle import sampler as O
+    from vllm_webgpu_amd import _lib
+
+    rng = np.random.default_rng(V)
+    B = 6
+    x = (rng.normal(size=(B, V)) * 3).astype(np.float32)
+    x[1, ::7] = -np.inf
+    x[1, V // 2] = 1.0
+    x[2, V // 3] = np.nan if V > 3 else 0.5
+    x[3, :] = -np.inf
+    x[3, min(77, V - 1)] = 2.5
+    x[4] = np.sort(x[4])
+    T = np.array([1.0, 0.7, 1.5, 1.0, 0.9, 3.0], np.float32)
+    t, Td = torch.from_numpy(x).to(cuda), torch.from_numpy(T).to(cuda)
+    out = t if inplace else torch.empty_like(t)
+    rm, ls = torch.empty(B, device=cuda), torch.empty(B, device=cuda)
+    _lib.check(_lib.lib().vws_softmax(t.data_ptr(), _lib.DTYPE_F32, B, V, V, Td.data_ptr(), out.data_ptr(),
+                                      rm.data_ptr(), ls.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    p, rm, ls = out.cpu().numpy(), rm.cpu().numpy(), ls.cpu().numpy()
+    for b in range(B):
+        rp, rrm, rls = O.softmax(x[b:b + 1], float(T[b]))
+        # the same exponentials as the oracle's, their sum in another order and its reciprocal once
+        np.testing.assert_allclose(p[b], rp[0], rtol=1e-6, atol=1e-12)
+        assert rm[b] == rrm[0]
+        np.testing.assert_allclose(ls[b], rls[0], rtol=1e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("kind", ["noise", "ties", "constant", "sparse"])
 @pytest.mark.parametrize("B,V,k", [(1, 7, 7), (3, 257, 256), (3, 4097, 1), (16, 128257, 20), (9, 70001, 100),

@@ -349,7 +349,7 @@ PROFILE_SUMMARIES = {1: "sample_c1_b1_v32000.md", 2: "sample_c2_b64_v32000.md",
 
 
 def pmc_traffic_bytes(config: int):
-    """HBM bytes per row_kernel launch from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary
+    """HBM bytes per sampling launch from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE summary
     (copy-calibrated); None when no summary covers this workload."""
     name = PROFILE_SUMMARIES.get(config)
     if name is None:
@@ -359,7 +359,7 @@ def pmc_traffic_bytes(config: int):
         text = open(path).read()
     except OSError:
         return None
-    m = re.search(r"^\| `void vws::row_kernel<[a-z0-9 ,]+>\([^`]*` \|(?:[^|\n]*\|){5} *([0-9.]+) *\|$",
+    m = re.search(r"^\| `void vws::(?:row|plain)_kernel<[a-z0-9 ,]+>\([^`]*` \|(?:[^|\n]*\|){5} *([0-9.]+) *\|$",
                   text, re.M)
     return None if m is None else float(m.group(1)) * 1e6
 
@@ -663,8 +663,9 @@ def main():
             "bound": "hbm", "achieved": gbps_kern, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
             "frac": gbps_kern / PEAK_HBM_GBPS, "traffic": pmc_traffic_bytes(args.config),
             # the instantiation the launch ran: element type, raw logprobs, logit transform
-            # (0: none; the bench's workloads have no allowed mask and no soft cap)
-            "kernel": "vws::row_kernel<{}, {}, 0>".format(
+            # (0: none; the bench's workloads have no allowed mask and no soft cap); config 1's
+            # greedy row is split over workgroups of the plain rows' kernel
+            "kernel": "vws::plain_kernel<float>" if args.config == 1 else "vws::row_kernel<{}, {}, 0>".format(
                 "unsigned short" if w.dtype == "bf16" else "float",
                 "true" if w.num_logprobs is not None else "false"),
         },

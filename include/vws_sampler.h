@@ -192,9 +192,11 @@ const char* vws_last_error(void);
  * which the workgroups of one launch share the extra passes over a row's logits that some
  * top-p rows need, and through which a batch larger than the device's resident workgroups
  * gets its rows handed out; then the history hash of rows served by the multi-pass path,
- * B x (power of two >= 2 x history_width, at least 64) x 16 bytes.  Every operation's
- * workspace starts with that same region (the others leave it alone), so one buffer can serve
- * them all in stream order. */
+ * B x (power of two >= 2 x history_width, at least 64) x 16 bytes.  The fixed region also holds
+ * what split rows count their parts with (temperature-only and greedy rows, the top-k operation).
+ * Every operation's workspace starts with that same region and leaves it clean, whatever its
+ * batch, so one buffer can serve them all in stream order; calls that may overlap (streams
+ * without an order between them, a graph's replays beside eager calls) need a buffer each. */
 size_t vws_sample_workspace_size(int32_t batch, int32_t vocab, int32_t history_width);
 
 /* Clears a workspace on `stream` (a fill kernel, safe under graph capture).  Required once
@@ -213,9 +215,10 @@ int vws_sample(const vws_sample_args* args);
 /* vws_sample without a caller workspace, for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart
  * in the reference.  `workspace` and `workspace_bytes` are ignored: the scratch is a static
- * device array of VWS_NOALLOC_SCRATCH_BYTES per GPU, looked up and cleared on the first call on
- * each device and held until the process ends.  Batches whose vws_sample_workspace_size exceeds
- * it are rejected with VWS_ERR_LIMIT.  Every call on one GPU shares that GPU's scratch: calls
+ * device array per GPU, looked up and cleared on the first call on each device and held until
+ * the process ends.  It holds every batch whose vws_sample_workspace_size is at most
+ * VWS_NOALLOC_SCRATCH_BYTES (and a little more: the array is that and 200 KiB of the fixed
+ * region); larger ones are rejected with VWS_ERR_LIMIT.  Every call on one GPU shares that GPU's scratch: calls
  * that overlap on one GPU (different streams, no ordering between them) race; calls ordered on
  * one stream do not.  Nothing is allocated, on the host or the device. */
 #define VWS_NOALLOC_SCRATCH_BYTES (16 << 20)

@@ -169,8 +169,8 @@ def test_repeat_calls_stable(cuda):
 
 
 def test_workspace_clean_after_general_path(cuda):
-    """The multi-pass path keeps its history hash in the shared workspace; it must leave zeros
-    behind, since the top-k operation's part counters overlap that region."""
+    """The multi-pass path keeps its history hash in the shared workspace and leaves zeros behind:
+    a top-k on the same buffer after it (whose part counters the hash once overlapped)."""
     import torch
 
     from tests.cases import _wl

@@ -38,8 +38,8 @@ using namespace vws;
 // Static device scratch of vws_sample_noalloc (one copy per GPU, held until the process ends).
 // Host code never uses this name as an address: the per-device address comes from
 // hipGetSymbolAddress (scratch_address below) and only that pointer is handed to kernels.
-// The plain rows' records and the top-k's counters come on top of the documented size, so that
-// they leave the accepted batches as they are.
+// The plain rows' records and the top-k's counters came into the fixed region later: they come on
+// top of the documented size, so that they leave the accepted batches as they are.
 constexpr size_t kExtraBytes = sizeof(CoopState::plain_ctr) + sizeof(CoopState::plain_rec) +
                                sizeof(CoopState::topk_ctr) + sizeof(CoopState::topk_state);
 constexpr size_t kScratchBytes = VWS_NOALLOC_SCRATCH_BYTES + kExtraBytes;
@@ -327,8 +327,8 @@ bool plain_launch(const vws_sample_args* a) {
 }
 
 // Parts per plain row: of at least 4096 tokens, four workgroups (of four waves) for each compute
-// unit: one round of the chip (128 x 151936 bf16: 3 / 4 / 5 / 7 / 8 workgroups 35.1 / 33.5 / 32.9 /
-// 36.2 / 39.3 us; 256 x 151936 fp32 with given uniforms 62.6 / 56.1 / 56.7 / 71.0 / 70.9 us); one
+// unit: one round of the chip (128 x 151936 bf16: 3 / 4 / 5 / 7 / 8 workgroups 31.6 / 30.8 / 35.7 /
+// 36.3 / 37.5 us; 256 x 151936 fp32 with given uniforms 63.0 / 55.7 / 75.1 / 64.2 / 63.3 us); one
 // part per row without the workspace or when the rows exceed its records.
 int plain_parts(const vws_sample_args* a, const void* ws) {
     if (!ws) return 1;
@@ -437,12 +437,14 @@ int vws_sample(const vws_sample_args* a) {
     if (plain_launch(a)) {
         void* ws = sample_workspace(a, hw);
         const int s = plain_parts(a, ws);
-        // All-greedy launches: the row kernel gives each row 1024 threads and one compute unit, so
-        // it stays for more than half the compute units' number of rows up to that number (one
-        // nearly full round: 256 x 128256 fp32 / bf16 26.1 / 18.5 us, here 27.7 / 21.2) and for few
-        // rows that are not split.  Otherwise (row kernel, here): 1 x 262144 bf16 17.7, 12.8 us;
-        // 128 x 151936 bf16 17.0, 16.3; 270 x 151936 fp32 56, 32.7; 400 x 32000 fp32 35, 15.3;
-        // 1000 x 6001 fp32 62, 12.8; 1024 x 128256 fp32 118, 81.
+        // All-greedy launches, a prepared call on the row kernel and here: 1 x 8192 fp32 11.6, 4.6 us;
+        // 1 x 32000 bf16 11.0, 5.5; 1 x 262144 bf16 17.8, 6.4; 128 x 151936 bf16 16.6, 12.6; 270 x
+        // 151936 fp32 56, 27.3; 400 x 32000 fp32 34.9, 10.8; 1000 x 6001 fp32 62, 6.2; 1024 x 128256
+        // fp32 111, 77.  The row kernel (1024 threads and one compute unit a row) keeps more than
+        // half the compute units' number of rows up to that number, and few rows that are not
+        // split: the line lay there when a nearly full round of it took 26.1 us (256 x 128256
+        // fp32) against 27.7 here; it takes 25.8 against 22.3 now, and 100 x 6001 12.0 against 5.0,
+        // so moving the line would pay (16-bit rows of a full round 16.6 on both).
         const int cus = device_info().cus, B = a->batch;
         if (a->temperature || B > 2 * cus || (s > 1 && (B <= cus / 2 || B > cus))) return sample_plain(a, ws, s);
     }

@@ -946,8 +946,7 @@ logprobs:
             fill_rest((int)n);
         }
     }
-    // the workspace is left as it was found (zeros): other operations that share it, such as
-    // the top-k's part counters, overlap the hash region
+    // the workspace is left as it was found (zeros)
     if (hh) {
         __syncthreads();
         for (int i = tid; i < hs; i += NT) { hkey[i] = 0u; hval[i] = 0u; hpen[i] = 0u; hadj[i] = 0u; }

@@ -307,7 +307,9 @@ int vws_profile_end(double* ms, int32_t* count);
  * and keeps alive): s_memrealtime stamps (a 100 MHz device clock) at the phase boundaries
  * below, by the first thread of the workgroup's last wave, and the XCD and row the workgroup
  * ran.  Each stamp delays the stamping wave by the clock read (the trace build's launches take
- * a few percent longer than the product build's).  A phase a
+ * a few percent longer than the product build's).  A row split over several workgroups
+ * (temperature-only and greedy rows) has a record of each, without the phases between its
+ * entry, its stream's end and the row.  A phase a
  * row does not reach keeps whatever the buffer held (clear it first).  vws_trace_set(NULL, 0)
  * turns it off.  Launches that overlap on one buffer overwrite each other's records. */
 #define VWS_TRACE_SLOTS 16

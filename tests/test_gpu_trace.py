@@ -44,6 +44,15 @@ def test_trace_records_and_results(cuda):
             assert (r[on, s0] > 0).all() and (r[on, s1] >= r[on, s0]).all(), (s0, s1)
     assert "top-p: masses -> cut decided" in trace.report(rec5, fl5, (1.0, 1.0), "C5", B5)
 
+    # a split greedy row: its workgroups record their entry, stream and end
+    rec1, fl1, kus1, name1, B1 = trace.collect(1, launches=3, warmup=1)
+    for i in range(3):
+        e, s, row, x = (rec1[i][:, k] for k in (_lib.TRACE_ENTRY, _lib.TRACE_STREAM, _lib.TRACE_ROW,
+                                                _lib.TRACE_EXIT))
+        assert (e > 0).all() and (s >= e).all() and (row >= s).all() and (x >= row).all()
+        assert (rec1[i][:, _lib.TRACE_ROWID] == 0).all()
+    assert "every wave streamed" in trace.report(rec1, fl1, kus1, name1, B1)
+
     # the same tokens from both builds
     w, xs, kw, _ = trace._inputs(2, cuda, False, 1)
     a = ops.sample(xs[0], **kw).sampled.cpu().numpy()

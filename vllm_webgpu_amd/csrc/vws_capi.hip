@@ -359,6 +359,13 @@ int sample_plain(const vws_sample_args* a, void* ws, int s) {
         k.rec = st->plain_rec;
         k.ctr = st->plain_ctr;
     }
+#ifdef VWS_TRACE
+    {
+        std::lock_guard<std::mutex> lock(g_trace_mu);
+        k.trace = g_trace_buf;
+        k.trace_wgs = g_trace_wgs;
+    }
+#endif
     const int nblk = a->vocab / 4;
     k.part_blocks = (nblk + s - 1) / s;
     k.S = k.part_blocks > 0 ? (nblk + k.part_blocks - 1) / k.part_blocks : 1;

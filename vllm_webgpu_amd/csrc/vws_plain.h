@@ -24,6 +24,10 @@ struct PlainArgs {
     int part_blocks;             // blocks of four tokens per part
     uint64_t* rec;               // [rows * S][8] (CoopState::plain_rec)
     uint32_t* ctr;               // [rows], left at zero
+#ifdef VWS_TRACE
+    uint64_t* trace;             // as KArgs::trace
+    int trace_wgs;
+#endif
 };
 
 __device__ __forceinline__ uint32_t tp_first(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }

@@ -315,6 +315,9 @@ __device__ __noinline__ void exact_row(uint64_t kernarg, int r, uint32_t maxk) {
 
 template <typename T>
 __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
+#ifdef VWS_TRACE
+    const uint64_t tr_entry = trace_clock();
+#endif
     PlainSmem& sm = g_plain_sh;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -327,6 +330,15 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
     const uint64_t seed = gen ? (a.rng_seed ? a.rng_seed[r] : a.rng_key) : 0ull;
     const uint64_t off = a.rng_seed ? (a.rng_offset ? a.rng_offset[r] : 0ull) : (uint64_t)(uint32_t)r;
     const float* urow = gen ? nullptr : a.u + (size_t)r * a.ustride;
+    auto traced = [&]() {  // trace build: the workgroup's record
+#ifdef VWS_TRACE
+        trace_mark(a, VWS_TRACE_ROW);
+        trace_put(a, VWS_TRACE_ENTRY, tr_entry);
+        trace_put(a, VWS_TRACE_XCC, trace_xcc());
+        trace_put(a, VWS_TRACE_ROWID, (uint64_t)r);
+        trace_mark(a, VWS_TRACE_EXIT);
+#endif
+    };
     // blocks of four tokens [b0, b1); the V % 4 tokens past the last block are thread 0's of the
     // last part
     const int nblk = a.V >> 2;
@@ -500,6 +512,7 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
         if (!greedy) race4(x, v, u, (uint32_t)t0, lane == 0);
     }
 
+    VWS_TRACE_MARK(a, VWS_TRACE_STREAM);
     // the part's record
     const uint32_t wk = wave_max_u32(key_of(mx));
     const uint64_t wg = wave_max_u64(gbest);
@@ -541,7 +554,10 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
         __syncthreads();
         if (tid == 0) sm.last = ag_add32(&a.ctr[r], 1u) == (uint32_t)(S - 1) ? 1u : 0u;
         __syncthreads();
-        if (!sm.last) return;
+        if (!sm.last) {
+            traced();
+            return;
+        }
         if (tid == 0) ag_store32(&a.ctr[r], 0u);
         for (int i = tid; i < S * 8; i += kPlThreads) sm.recs[i >> 3][i & 7] = ag_load64(rec + i);
         __syncthreads();
@@ -554,6 +570,7 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
             const bool any = (best >> 32) != 0ull;  // (an element that is not NaN)
             plain_write(a, r, any ? (int32_t)(0x7FFFFFFFu - (uint32_t)best) : 0, VWS_FLAG_GREEDY, 1);
         }
+        traced();
         return;
     }
     uint32_t maxk = 0u, count = 0u, over = 0u, ntot = 0u;
@@ -598,6 +615,7 @@ __global__ __launch_bounds__(kPlThreads) void plain_kernel(PlainArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     if (exact) exact_row<T>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr(), r, maxk);
 #endif
+    traced();
 }
 
 template __global__ void plain_kernel<float>(PlainArgs);

@@ -15,14 +15,17 @@ namespace vws {
 // VWS_TRACE_MARK_AFTER first waits for dep, a value the phase produced, so that the stamp
 // cannot be taken before the phase's loads have landed.
 #ifdef VWS_TRACE
-__device__ __forceinline__ bool trace_lane(const KArgs& a) {
+template <typename A>
+__device__ __forceinline__ bool trace_lane(const A& a) {
     return a.trace && threadIdx.x == blockDim.x - 64u && (int)blockIdx.x < a.trace_wgs;
 }
-__device__ __forceinline__ void trace_put(const KArgs& a, int s, uint64_t v) {
+template <typename A>
+__device__ __forceinline__ void trace_put(const A& a, int s, uint64_t v) {
     if (trace_lane(a)) a.trace[(size_t)blockIdx.x * VWS_TRACE_SLOTS + s] = v;
 }
 // the clock is read by the stamping wave alone (the others issue nothing)
-__device__ __forceinline__ void trace_mark(const KArgs& a, int s) {
+template <typename A>
+__device__ __forceinline__ void trace_mark(const A& a, int s) {
     if (trace_lane(a)) a.trace[(size_t)blockIdx.x * VWS_TRACE_SLOTS + s] = __builtin_amdgcn_s_memrealtime();
 }
 __device__ __forceinline__ uint64_t trace_clock() { return __builtin_amdgcn_s_memrealtime(); }

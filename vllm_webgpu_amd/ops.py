@@ -115,8 +115,9 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     torch's allocator, which hands it out again in the order of the stream that used it.
 
     Under graph capture each call gets a buffer that nothing else uses and that the graph clears:
-    a replay may overlap any stream's eager calls.  Its memory is the capture's (torch gives the
-    allocations of a capture to the graph's own pool), not the cache's.
+    a replay may overlap any stream's eager calls.  Its memory is the capture's, not the cache's:
+    torch gives what is allocated under its own captures (``torch.cuda.graph``) to the graph's
+    pool, which lives as long as the graph.
     """
     idx = device.index if device.index is not None else torch.cuda.current_device()
     stream = torch._C._cuda_getCurrentRawStream(idx)
